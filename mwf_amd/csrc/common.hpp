@@ -73,7 +73,7 @@ struct Geo {
     int NTs;           // z-modes per NL piece (a multiple of NTx, power of two)
     int lgNS;          // log2(NTs)
     int XB;            // x-rows per z-kernel block
-    int UL, NLL;       // lines per x-row of U and NL: 2 KK and KK (advective form), KK and 2 KK (flux form)
+    int UL, NLL;       // lines per x-row of U and NL: 2 KK and KK (advective form), KK and 4 K0 - 2 (flux form)
     double alpha, gamma, re, dt, drag, vdrag, hypo, cth, sth, beta;
     double scale;      // 1/(P*Q), transform.fftw5.f90:242
     int dragall;
@@ -132,3 +132,9 @@ __device__ __forceinline__ size_t nidx(const Geo& g, int x, int slot, int n)
 // wall-normal derivative table ad_k1, ad_k2 (program/variables.f90:528-531)
 __device__ __forceinline__ double ak1_of(int k, double beta) { return ((k & 1) ? -1.0 : 1.0) * k * beta; }
 __device__ __forceinline__ double ak2_of(int k, double beta) { return -k * k * beta * beta; }
+
+// Lines of NL in the flux form (zflux.hpp): per wall-normal index k >= 1 uw,
+// F, uv, E, for k = 0 uw and F.
+enum { DEV_UW, DEV_F, DEV_UV, DEV_E };
+__host__ __device__ constexpr int dev_line(int k) { return k == 0 ? 0 : 4 * k - 2; }
+__host__ __device__ constexpr int dev_lines(int K0) { return 4 * K0 - 2; }

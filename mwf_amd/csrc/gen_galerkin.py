@@ -39,9 +39,9 @@ spectral space:
   uu_i = P_h,i(u u), uw_i = P_h,i(u w), ww_i = P_h,i(w w)   (i < K0)
   uv_i = P_g,i(u v), vw_i = P_g,i(v w), vv_i = P_h,i(v v)   (1 <= i < K0)
 
-The z kernel of this form transforms the rows forward and emits, per spec
-slot s, a line B_s to be differentiated in x (uu, uv, uw) and a line A_s
-(the d/dy and d/dz terms); the x kernel forms N_s = i alpha m B_s + A_s.
+The z kernel of this form needs only the rows of dev_rows (five per i >= 1): the
+step takes the nonlinear term as its psi and phi parts, and in those the
+products' trace drops out (zflux.hpp has the algebra).
 
 Run:  python mwf_amd/csrc/gen_galerkin.py   (rewrites galerkin_gen.hpp and flux_gen.hpp)
 """
@@ -229,18 +229,6 @@ def flux_rows(k0):
     return rows
 
 
-def flux_order(k0):
-    """Forward order of the rows (indices into flux_rows): i = 0 first, then per
-    i the rows of one wall-normal index together, so that partial lines live
-    briefly."""
-    rows = flux_rows(k0)
-    idx = {(n, i): r for r, (n, i, _) in enumerate(rows)}
-    order = [idx[("uu", 0)], idx[("uw", 0)], idx[("ww", 0)]]
-    for i in range(1, k0):
-        order += [idx[(n, i)] for n in ("uv", "uw", "vw", "ww", "uu", "vv")]
-    return order
-
-
 def ak1_sign(i):
     """ak1(i) / beta = (-1)^i i (program/variables.f90:528-529)."""
     return (-1) ** i * i
@@ -271,52 +259,65 @@ def flux_lines(k0):
     return lines
 
 
+def dev_rows(k0):
+    """Real rows of the flux form's z pass in forward order: (name, terms).  Of
+    the six products of a wall-normal index the psi and phi parts of the
+    nonlinear term take only the trace-free part, so uu, vv and ww enter as two
+    differences (for i = 0, with no vv, as one)."""
+    prods = {(n, i): t for n, i, t in flux_rows(k0)}
+
+    def diff(a, b, i):
+        acc = {}
+        for terms, sg in ((prods[(a, i)], 1), (prods[(b, i)], -1)):
+            for x, y, c in terms:
+                acc[(x, y)] = acc.get((x, y), F(0)) + sg * c
+        return sorted((x, y, c) for (x, y), c in acc.items() if c != 0)
+
+    rows = [("uw_0", prods[("uw", 0)]), ("ww_0 - uu_0", diff("ww", "uu", 0))]
+    for i in range(1, k0):
+        rows += [(f"uv_{i}", prods[("uv", i)]), (f"uw_{i}", prods[("uw", i)]),
+                 (f"vv_{i} - uu_{i}", diff("vv", "uu", i)), (f"vw_{i}", prods[("vw", i)]),
+                 (f"vv_{i} - ww_{i}", diff("vv", "ww", i))]
+    return rows
+
+
 def emit_flux(k0s=(4, 6)):
     out = [
         "// GENERATED by gen_galerkin.py -- do not edit.",
-        "// Flux (conservative) form of the wall-normal Galerkin products: the",
-        "// projected product rows uu, uw, ww, uv, vw, vv of the base values and",
-        "// how the z kernel assembles them into the B (d/dx) and A (d/dy + d/dz)",
-        "// lines; see gen_galerkin.py for the derivation.",
+        "// Flux (conservative) form of the wall-normal Galerkin products: the real",
+        "// rows of the z pass at one point, from the base values v[KK] of the",
+        "// perturbation and the laminar profile (lu, lw) sin(beta y), which adds lu to",
+        "// u_1 and lw to w_1.  The constants of the profile's own products (lu lu, lu",
+        "// lw, lw lw) are left out: they touch the (0,0) mode of uw, ww - uu and vv - uu",
+        "// only, which nothing reads.  See gen_galerkin.py for the derivation.",
         "#pragma once",
         "",
-        "template <int K0> struct Flux;",
+        "template <int K0> struct FluxRows;",
         "",
     ]
     for k0 in k0s:
-        rows, order, lines = flux_rows(k0), flux_order(k0), flux_lines(k0)
-        kk, nr = 3 * k0 - 1, len(rows)
-        pos = {r: q for q, r in enumerate(order)}
-        uses = [[] for _ in range(nr)]
-        for L, terms in enumerate(lines):
-            for r, kind, sg in terms:
-                uses[r].append((L, kind, sg))
-        last = [max(pos[r] for r, _, _ in lines[L]) for L in range(2 * kk)]
-        first = [min(pos[r] for r, _, _ in lines[L]) for L in range(2 * kk)]
-        arr = lambda v: "{" + ", ".join(str(x) for x in v) + "}"
-        out.append(f"template <> struct Flux<{k0}> {{")
-        out.append(f"  static constexpr int KK = {kk};")
-        out.append(f"  static constexpr int NR = {nr};  // product rows")
-        out.append("  // row at forward position q (two rows per complex sequence); -1 = padding")
-        out.append(f"  __host__ __device__ static constexpr int order(int q) {{ constexpr int o[] = {arr(order)}; "
-                   f"return q < NR ? o[q] : -1; }}")
-        out.append("  // uses of row r: line, kind (0: +row, 1: + s beta row, 2: + i gamma n row), s")
-        out.append(f"  __host__ __device__ static constexpr int nuse(int r) {{ constexpr int o[] = {arr(len(u) for u in uses)}; return o[r]; }}")
-        for nm, j in (("use_line", 0), ("use_kind", 1), ("use_sign", 2)):
-            flat = [u[k][j] if k < len(u) else 0 for u in uses for k in range(2)]
-            out.append(f"  __host__ __device__ static constexpr int {nm}(int r, int u) {{ constexpr int o[] = {arr(flat)}; "
-                       f"return o[2 * r + u]; }}")
-        out.append("  // forward position of the last row of line L (the line is complete after it)")
-        out.append(f"  __host__ __device__ static constexpr int last(int L) {{ constexpr int o[] = {arr(last)}; return o[L]; }}")
-        out.append("  // forward position of the first row of line L (the line starts there)")
-        out.append(f"  __host__ __device__ static constexpr int first(int L) {{ constexpr int o[] = {arr(first)}; return o[L]; }}")
-        out.append("  // value of product row ROW from the base values v[KK] of one point")
+        u1, w1 = 1, 2 * k0
+
+        def val(s):
+            return {u1: "u1", w1: "w1"}.get(s, f"v[{s}]")
+
+        def term(a, b, c):
+            if a == b and a in (u1, w1):  # (l + v)^2 - l^2
+                m = f"(v[{a}] * ({val(a)} + {'lu' if a == u1 else 'lw'}))"
+            elif (a, b) == (u1, w1):      # (lu + u)(lw + w) - lu lw
+                m = f"(v[{a}] * w1 + lu * v[{b}])"
+            else:
+                m = f"({val(a)} * {val(b)})"
+            return m if c == 1 else f"(R){lit(c)} * {m}"
+
+        rows = dev_rows(k0)
+        out.append(f"template <> struct FluxRows<{k0}> {{")
         out.append("  template <int ROW, typename R>")
-        out.append("  __host__ __device__ static __forceinline__ R row(const R* v) {")
-        for r, (name, i, terms) in enumerate(rows):
+        out.append("  __host__ __device__ static __forceinline__ R row(const R* v, R lu, R lw) {")
+        out.append(f"    const R u1 = v[{u1}] + lu, w1 = v[{w1}] + lw;")
+        for r, (name, terms) in enumerate(rows):
             kw = "if constexpr" if r == 0 else "else if constexpr"
-            expr = " + ".join(("" if c == 1 else f"(R){lit(c)} * ") + f"(v[{a}] * v[{b}])" for a, b, c in terms)
-            out.append(f"    {kw} (ROW == {r}) {{ return {expr or '(R)0'}; }}  // {name}_{i}")
+            out.append(f"    {kw} (ROW == {r}) {{ return {' + '.join(term(*t) for t in terms)}; }}  // {name}")
         out.append("    else { return (R)0; }")
         out.append("  }")
         out.append("};")

@@ -166,7 +166,8 @@ __global__ __launch_bounds__(XT) void k_xinv(Batch bt, const double2* __restrict
                     }
                 }
             }
-            if (addlam) mpt2spec_k(g, k, mi, n, psi, phi, true, u, v, w);
+            // the flux form's U holds the perturbation alone
+            if (addlam && !FLUX) mpt2spec_k(g, k, mi, n, psi, phi, true, u, v, w);
             sp[q][h][0] = u;
             sp[q][h][1] = v;
             sp[q][h][2] = w;
@@ -396,15 +397,15 @@ __device__ __forceinline__ void zfold_b(cplx_t<R>* __restrict__ seq, int b, int 
 }
 
 // w^k = exp(2 pi i k/Q), Q = 3 NN, for 0 <= k < 2 NN from a table of the
-// first NN entries: w^{NN + j} = exp(2 pi i/3) w^j.
+// first NN entries, exactly: with j = k - Q/2, w^k = -w^j, and w^j = conj(w^-j).
 template <typename R>
 __device__ __forceinline__ cplx_t<R> twq2(const cplx_t<R>* __restrict__ tw, int NN, int k)
 {
     using CT = cplx_t<R>;
     if (k < NN) return tw[k];
-    const CT w = tw[k - NN];
-    const R c = (R)-0.5, sn = (R)0.86602540378443864676; // exp(2 pi i/3)
-    return CT{c * w.x - sn * w.y, c * w.y + sn * w.x};
+    const int j = k - (NN + NN / 2);
+    const CT w = tw[j < 0 ? -j : j];
+    return CT{-w.x, j < 0 ? w.y : -w.y};
 }
 
 // two transform buffers, then the pass twiddle table of the NN-point
@@ -1118,6 +1119,41 @@ __device__ __forceinline__ void s2m_finish(int k, int mi, int n, double2 u, doub
     }
 }
 
+// Flux form: the share of line type li (uw, F, uv, E of wall-normal index k,
+// zflux.hpp; not yet scaled by 1/(PQ)) in psi_k and phi_k of the nonlinear term
+// at one (m, n), from the line's forward x transform X; rak = 1/ak1, for k = 0
+// -1 (F_0 has the multiplier a).  At (0,0), where every multiplier vanishes, the
+// mean-mode rows of var_spec2mpt apply instead: psi = -N_u = -ak uv, phi = -N_w =
+// i F / ak.
+__device__ __forceinline__ void dev_term(int li, bool mean, double2 X, double am1, double an1, double ak1, double rak,
+                                         double2& psi, double2& phi)
+{
+    if (li == DEV_UV) X = double2{-X.y, X.x}; // i uv
+    const double a2 = am1 * am1, g2 = an1 * an1;
+    double cp, cq;
+    if (li == DEV_UW) {
+        cp = a2 - g2;
+        cq = -2.0 * ak1 * (am1 * an1);
+    } else if (li == DEV_F) {
+        cp = -(am1 * rak);
+        cq = an1;
+    } else if (li == DEV_UV) {
+        cp = an1 * ak1;
+        cq = am1 * (ak1 * ak1 - (a2 + g2));
+    } else {
+        cp = am1 * an1 * rak;
+        cq = a2;
+    }
+    psi.x += cp * X.x;
+    psi.y += cp * X.y;
+    phi.x += cq * X.x;
+    phi.y += cq * X.y;
+    if (mean) {
+        if (li == DEV_UV) psi = double2{-(ak1 * X.y), ak1 * X.x}; // -ak uv, X = i uv
+        if (li == DEV_F) phi = double2{-(X.y * rak), X.x * rak};
+    }
+}
+
 // var_LHSRHS (program/variables.f90:565-597) for psi_k (which = 0) or
 // phi_k (which = 1) at one (m, n).
 __device__ __forceinline__ void lhsrhs_k(const Geo& g, int k, int which, bool mean, double am2, double an2,
@@ -1209,18 +1245,16 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
     const int k = blockIdx.y;
     const int tid = threadIdx.x;
     const int nitems = NT * MM;
-    const double ak1 = ak1_of(k, g.beta);
+    const double ak1 = ak1_of(k, g.beta), rak = k == 0 ? -1.0 : 1.0 / ak1;
 
-    // psi[] holds u_k until w_k arrives, phi[] holds v_k (am2+an2) until then;
-    // xd[] holds i alpha m B of the flux form until its A line arrives
-    double2 psi[IPT][2], phi[IPT][2];
-    double2 xd[FLUX ? IPT : 1][2];
+    // flux form: psi[] and phi[] sum the lines' shares; otherwise psi[] holds
+    // u_k until w_k arrives, phi[] holds v_k (am2+an2) until then
+    double2 psi[IPT][2] = {}, phi[IPT][2] = {};
 
-    for (int li = 0; li < (FLUX ? 6 : 3); li++) {
-        const int comp = FLUX ? li >> 1 : li, part = FLUX ? li & 1 : 0;
-        if (k == 0 && comp == 1) continue;
-        const int slot = comp == 0 ? k : (comp == 1 ? g.K0 - 1 + k : 2 * g.K0 - 1 + k);
-        const CT* pan = nl_panel(g, NL, n0, slot + part * g.KK);
+    for (int li = 0; li < (FLUX ? 4 : 3); li++) {
+        if (k == 0 && (FLUX ? li > DEV_F : li == 1)) continue;
+        const int slot = FLUX ? dev_line(k) + li : (li == 0 ? k : (li == 1 ? g.K0 - 1 + k : 2 * g.K0 - 1 + k));
+        const CT* pan = nl_panel(g, NL, n0, slot);
         // load NL rows, decimated by b = x mod 3
 #pragma unroll
         for (int q = 0; q < 3 * IPT; q++) {
@@ -1270,18 +1304,15 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
                 double am1, am2, an1, an2;
                 xwave(g, mi, am1, am2);
                 zwave(g, n, an1, an2);
-                double2 X = X0;
-                if constexpr (FLUX) { // N = i alpha m B + A
-                    if (part == 0) {
-                        xd[q][h] = double2{-(X.y * am1), X.x * am1};
-                        continue;
-                    }
-                    X = double2{xd[q][h].x + X.x, xd[q][h].y + X.y};
+                const double2 X = X0;
+                if constexpr (FLUX) {
+                    dev_term(li, mi == 0 && n == 0, X, am1, an1, ak1, rak, psi[q][h], phi[q][h]);
+                    continue;
                 }
                 // var_spec2mpt (program/variables.f90:440-480)
-                if (comp == 0) {
+                if (li == 0) {
                     psi[q][h] = X;
-                } else if (comp == 1) {
+                } else if (li == 1) {
                     phi[q][h] = s2m_vterm(X, am2, an2);
                 } else {
                     const double2 u = psi[q][h], vh = phi[q][h];
@@ -1315,7 +1346,8 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
                 if (which == 1 && k == 0) continue;
                 const int slot = which == 0 ? k : g.K0 - 1 + k;
                 const size_t idx = ((size_t)n * g.K + slot) * g.ldM + mi;
-                const double2 nl = which == 0 ? psi[q][h] : phi[q][h];
+                double2 nl = which == 0 ? psi[q][h] : phi[q][h];
+                if constexpr (FLUX) nl = double2{nl.x * g.scale, nl.y * g.scale};
                 if (mode == 1) {
                     nlout[idx] = nl;
                     continue;
@@ -1453,14 +1485,13 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
         rb = reg + (t0 * 3 + b0) * MM;
         pa = pidx(a0) ^ xsw<R>(t0, b0);
     };
-    const double ak1 = ak1_of(k, g.beta);
+    const double ak1 = ak1_of(k, g.beta), rak = k == 0 ? -1.0 : 1.0 / ak1;
     const double ak2 = ak2_of(k, g.beta);
 
-    // psi[] holds u_k until w_k arrives, phi[] holds v_k (am2+an2); after the
-    // update both hold the new state.  xd[] holds i alpha m B of the flux
-    // form until its A line arrives.
-    double2 psi[IPT][2], phi[IPT][2];
-    double2 xd[FLUX ? IPT : 1][2];
+    // flux form: psi[] and phi[] sum the lines' shares; otherwise psi[] holds
+    // u_k until w_k arrives, phi[] holds v_k (am2+an2).  After the update both
+    // hold the new state.
+    double2 psi[IPT][2] = {}, phi[IPT][2] = {};
 
     ptw_fill<CT, LOGMM, 1, 7>(twMl, twMM, tid, XS);
     for (int i = tid; i <= 2 * MM; i += XS) twPl[i] = twP[i];
@@ -1470,20 +1501,18 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
 
     if constexpr (!INV_ONLY) {
         // ---------------- forward x transform + spec2mpt ----------------
-        // NL lines in order: comp u, v, w (flux form: B then A of each);
-        // y-mode 0 has no v
-        constexpr int NLI = FLUX ? 6 : 3;
-        auto line_on = [&](int li) { return !(k == 0 && (FLUX ? li >> 1 : li) == 1); };
+        // NL lines in order: u, v, w (y-mode 0 has no v); flux form: uw, F,
+        // uv, E (y-mode 0: uw, F)
+        constexpr int NLI = FLUX ? 4 : 3;
+        auto line_on = [&](int li) { return !(k == 0 && (FLUX ? li > DEV_F : li == 1)); };
         auto panel_of = [&](int li) {
-            const int comp = FLUX ? li >> 1 : li, part = FLUX ? li & 1 : 0;
-            const int slot = comp == 0 ? k : (comp == 1 ? g.K0 - 1 + k : 2 * g.K0 - 1 + k);
-            return nl_panel(g, NL, n0, slot + part * g.KK);
+            const int slot = FLUX ? dev_line(k) + li : (li == 0 ? k : (li == 1 ? g.K0 - 1 + k : 2 * g.K0 - 1 + k));
+            return nl_panel(g, NL, n0, slot);
         };
         const int nch = nrows * (int)sizeof(CT) / 16; // 16-byte chunks of one stripe
         if constexpr (ASYNC) panel_to_lds<XS>(g, panel_of(0), stage, nch, tid);
 #pragma unroll 1
         for (int li = 0; li < NLI; li++) {
-            const int comp = FLUX ? li >> 1 : li, part = FLUX ? li & 1 : 0;
             if (!line_on(li)) continue;
             // opaque copy of the thread index: keeps item arithmetic inside the loop
             int tidv = tid;
@@ -1602,16 +1631,13 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
                     double am1, am2, an1, an2;
                     xwave(g, mi, am1, am2);
                     zwave(g, n, an1, an2);
-                    if constexpr (FLUX) { // N = i alpha m B + A
-                        if (part == 0) {
-                            xd[q][h] = double2{-(X.y * am1), X.x * am1};
-                            continue;
-                        }
-                        X = double2{xd[q][h].x + X.x, xd[q][h].y + X.y};
+                    if constexpr (FLUX) {
+                        dev_term(li, mi == 0 && n == 0, X, am1, an1, ak1, rak, psi[q][h], phi[q][h]);
+                        continue;
                     }
-                    if (comp == 0) {
+                    if (li == 0) {
                         psi[q][h] = X;
-                    } else if (comp == 1) {
+                    } else if (li == 1) {
                         phi[q][h] = s2m_vterm(X, am2, an2);
                     } else {
                         const double2 u = psi[q][h], vh = phi[q][h];
@@ -1643,7 +1669,8 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
                     if (which == 1 && k == 0) continue;
                     const int slot = which == 0 ? k : g.K0 - 1 + k;
                     const size_t idx = ((size_t)n * g.K + slot) * g.ldM + mi;
-                    const double2 nl = which == 0 ? psi[q][h] : phi[q][h];
+                    double2 nl = which == 0 ? psi[q][h] : phi[q][h];
+                    if constexpr (FLUX) nl = double2{nl.x * g.scale, nl.y * g.scale};
                     double lhs, rhs;
                     lhsrhs_k(g, k, which, mean, am2, an2, ak2, lhs, rhs);
                     const double2 cv = c[idx];
@@ -1698,7 +1725,7 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
                     if (k > 0) ph = cn[(size_t)(g.K0 - 1 + k) * g.ldM + mi];
                 }
                 double2 u, v, w;
-                mpt2spec_k(g, k, mi, n, ps, ph, true, u, v, w);
+                mpt2spec_k(g, k, mi, n, ps, ph, !FLUX, u, v, w);
                 double2 val = comp == 0 ? u : (comp == 1 ? v : w);
                 if (deriv) { // i alpha m (program/variables.f90:606-607)
                     double am1, am2;

@@ -220,8 +220,8 @@ struct SizeClass {
             return fail(MWF_E_ARG, "no kernel for this size");
         const size_t rsz = prec == MWF_MIXED ? sizeof(float2) : sizeof(double2);
         mpt_elems = (size_t)g0.NN * g0.K * g0.ldM;
-        // room for either form: U and NL each hold up to 2 KK lines per x-row
-        const size_t u_el = (size_t)g0.P * 2 * g0.KK * g0.NN, nl_el = (size_t)g0.P * 2 * g0.KK * g0.NN;
+        // room for either form: U holds up to 2 KK lines per x-row, NL dev_lines(K0) >= KK
+        const size_t u_el = (size_t)g0.P * 2 * g0.KK * g0.NN, nl_el = (size_t)g0.P * dev_lines(g0.K0) * g0.NN;
         nepart = (g0.NN / g0.NTx) * g0.K0;
         RCCHK(dev_upload(&geos, geos_h.data(), geos_h.size()));
         HIPCHK(hipMalloc((void**)&c, sizeof(double2) * mpt_elems * nmem));
@@ -276,7 +276,7 @@ struct SizeClass {
         // panels into LDS and takes them with the split x kernels
         if ((ch & 2) || (ph3 && prec == MWF_MIXED)) plan.xstep = nullptr;
         bt.nl_part = ph3 ? bt.nl_stride * nmem : 0;
-        const int UL = flux ? g0.KK : 2 * g0.KK, NLL = flux ? 2 * g0.KK : g0.KK;
+        const int UL = flux ? g0.KK : 2 * g0.KK, NLL = flux ? dev_lines(g0.K0) : g0.KK;
         if (g0.UL != UL) {
             g0.UL = UL;
             g0.NLL = NLL;

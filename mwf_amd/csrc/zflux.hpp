@@ -4,14 +4,29 @@
 // For the divergence-free Galerkin field, (u.grad)u = div(u u), and the
 // wall-normal derivative moves onto the bases exactly (gen_galerkin.py has
 // the derivation).  The z pass then needs only the KK base lines of U (u_k,
-// v_k, w_k; no x- or z-derivatives): per point it forms the 6 K0 - 3
-// projected products uu_i, uw_i, ww_i, uv_i, vw_i, vv_i (flux_gen.hpp),
-// transforms them forward, and writes per spec slot s a line B_s (to be
-// differentiated in x by the x kernel) and a line A_s = (ak1 terms) + i gamma
-// n (z terms).  NL thus holds 2 KK lines per x-row (B at line s, A at KK + s),
-// U only KK.  Compared with the advective z kernel this transforms
-// ceil(KK/2) + ceil(NR/2) pairs instead of ceil(3 KK/2) + ceil(KK/2) (M4: 17
-// against 23) and keeps KK values per point instead of 2 KK.
+// v_k, w_k; no x- or z-derivatives).  The step needs the nonlinear term only as
+// its psi and phi parts (var_spec2mpt), and of the six projected products
+// uu, uw, ww, uv, vw, vv of a wall-normal index k these take the trace-free
+// part alone (the trace is a pressure gradient).  With a = alpha m,
+// g = gamma n, ak = ak1(k):
+//
+//   E_k = ak (vv_k - uu_k) - i g vw_k
+//   F_k = ak g (vv_k - ww_k) + i (ak^2 - g^2) vw_k
+//   psi_k = (a^2 - g^2) uw_k + i g ak uv_k + (a g / ak) E_k - (a / ak) F_k
+//   phi_k = i a (ak^2 - a^2 - g^2) uv_k - 2 ak a g uw_k + a^2 E_k + g F_k
+//   psi_0 = (a^2 - g^2) uw_0 + a F_0,  F_0 = g (ww_0 - uu_0)
+//
+// so five real rows per k >= 1 (uv, uw, vv - uu, vw, vv - ww; two for k = 0) are
+// transformed forward, and four lines per k >= 1 (uw, F, uv, E; two for k = 0)
+// cross to the x kernel, which applies the powers of a and the scale 1/(PQ)
+// (Dev below, and dev_term in kernels.hpp): M4 17 rows and 14 lines, M6 27 and
+// 22.  The form with one line to be differentiated in x and one for the rest per
+// spec slot has 21 rows and 22 lines (33 and 34), so 36 % of NL's bytes and of
+// the forward x transforms are saved: at M4 1024^2 k_zc 157 -> 141 us and
+// k_xstep 192 -> 149 us in FP64, 79 -> 72 and 121 -> 101 us in FP32.
+// Of the equivalent pairs of lines this one keeps the largest products, uu, at
+// the weights a^2 and a g they have in the plain form (E and g (ww - uu) - i ak vw
+// would add a g^2), which the rounding of the FP32 form follows.
 //
 // Block: T = max(512, NN) threads, XB = T/NN x-rows; thread (xl, r) owns the
 // points z = 3r + b, b = 0..2, of row xl, and the output index n = r of that
@@ -28,6 +43,56 @@
 #pragma once
 #include "kernels.hpp"
 #include "flux_gen.hpp"
+
+// Rows and lines of the z pass.  Row r (value: FluxRows in flux_gen.hpp): 0, 1
+// are uw_0, ww_0 - uu_0; 2 + 5 (k-1) + t, t = 0..4, are uv, uw, vv - uu, vw, vv -
+// ww of k >= 1, transformed two per complex sequence in this order.  Lines of
+// k start at dev_line(k).
+//
+// U holds the perturbation; the laminar profile enters where the rows are
+// formed, without its own products, whose constants only the unused (0,0) modes
+// would see.  With the profile in U the rounding of its unit-size constant
+// spread over every mode: the FP32 nonlinear term is 1.5 to 6 times closer to
+// the FP64 one this way (rms velocity 0.3 to 0.05).
+template <int K0_> struct Dev {
+    static constexpr int K0 = K0_, KK = 3 * K0 - 1;
+    static constexpr int NR = 5 * K0 - 3;     // real rows
+    static constexpr int NL = dev_lines(K0);  // output lines
+    enum { UV, UW, VVUU, VW, VVWW, WWUU };
+    __host__ __device__ static constexpr int k(int r) { return r < 2 ? 0 : 1 + (r - 2) / 5; }
+    __host__ __device__ static constexpr int type(int r) { return r < 2 ? (r == 0 ? UW : WWUU) : (r - 2) % 5; }
+    __host__ __device__ static constexpr int order(int q) { return q < NR ? q : -1; }
+    // uses of row r: line, kind (0: row, 1: ak row, 2: g row, 3: -i g row, 4: ak g row, 5: i (ak^2 - g^2) row)
+    __host__ __device__ static constexpr int nuse(int r) { return type(r) == VW ? 2 : 1; }
+    __host__ __device__ static constexpr int use_line(int r, int u)
+    {
+        const int t = type(r);
+        return dev_line(k(r)) + (t == UW ? DEV_UW : t == UV ? DEV_UV : t == VVUU || (t == VW && u == 0) ? DEV_E : DEV_F);
+    }
+    __host__ __device__ static constexpr int use_kind(int r, int u)
+    {
+        const int t = type(r);
+        return t == VVUU ? 1 : t == WWUU ? 2 : t == VW ? (u == 0 ? 3 : 5) : t == VVWW ? 4 : 0;
+    }
+    // ak1(k) / beta = (-1)^k k (program/variables.f90:528-529)
+    __host__ __device__ static constexpr int sign(int r) { return (k(r) & 1) ? -k(r) : k(r); }
+    // forward positions of the first and the last row of line L
+    __host__ __device__ static constexpr int first(int L)
+    {
+        for (int r = 0; r < NR; r++)
+            for (int u = 0; u < nuse(r); u++)
+                if (use_line(r, u) == L) return r;
+        return -1;
+    }
+    __host__ __device__ static constexpr int last(int L)
+    {
+        int q = -1;
+        for (int r = 0; r < NR; r++)
+            for (int u = 0; u < nuse(r); u++)
+                if (use_line(r, u) == L) q = r;
+        return q;
+    }
+};
 
 template <int LOGNN> constexpr int zc_threads() { return (1 << LOGNN) > ZT ? (1 << LOGNN) : ZT; }
 
@@ -89,7 +154,8 @@ __global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, con
                                                                    const cplx_t<R>* __restrict__ twQ)
 {
     using CT = cplx_t<R>;
-    using FX = Flux<K0>;
+    using FX = Dev<K0>;
+    using FR = FluxRows<K0>;
     const Geo g = bt.geo[blockIdx.z];
     U += blockIdx.z * bt.u_stride;
     NL += blockIdx.z * bt.nl_stride;
@@ -234,10 +300,12 @@ __global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, con
     });
 
     // ---- products, forward z transforms (r2c, -1), line assembly ----
-    const R scale = (R)g.scale;
-    const R gn = (R)(g.gamma * r);       // i gamma n at the thread's output n = r
-    const R beta = (R)g.beta;
-    CT acc[2 * KK];
+    const R gn = (R)(g.gamma * r);       // gamma n at the thread's output n = r
+    const R beta = (R)g.beta, bg = (R)(g.beta * (g.gamma * r));
+    const R b2 = (R)(g.beta * g.beta), g2 = (R)((g.gamma * r) * (g.gamma * r));
+    const R lu = (R)g.cth, lw = (R)g.sth; // laminar u_1, w_1
+    constexpr int NLN = FX::NL;          // lines of NL
+    CT acc[NLN];
     // line assembly of the two rows q1, q1 + 1 of a forward pair from their
     // transforms X: each row's terms go into the accumulators of its lines,
     // and a line is stored after its last row
@@ -247,14 +315,20 @@ __global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, con
             constexpr int q = q1 + decltype(hi)::value;
             constexpr int row = FX::order(q);
             if constexpr (row >= 0) {
-                const CT xs = cscale(X[decltype(hi)::value], scale);
+                const CT xs = X[decltype(hi)::value];
                 static_for<0, FX::nuse(row)>([&](auto ui) {
                     constexpr int u = decltype(ui)::value;
                     constexpr int L = FX::use_line(row, u), kind = FX::use_kind(row, u);
-                    constexpr int sg = FX::use_sign(row, u);
+                    constexpr int sg = FX::sign(row);
                     CT term = xs;
                     if constexpr (kind == 1) term = cscale(xs, (R)sg * beta);
-                    else if constexpr (kind == 2) term = CT{-(xs.y * gn), xs.x * gn};
+                    else if constexpr (kind == 2) term = cscale(xs, gn);
+                    else if constexpr (kind == 3) term = CT{xs.y * gn, -(xs.x * gn)};
+                    else if constexpr (kind == 4) term = cscale(xs, (R)sg * bg);
+                    else if constexpr (kind == 5) {
+                        const R f = (R)(sg * sg) * b2 - g2;
+                        term = CT{-(xs.y * f), xs.x * f};
+                    }
                     if constexpr (FX::first(L) == q) acc[L] = term;
                     else acc[L] = cadd(acc[L], term);
                     if constexpr (FX::last(L) == q) {
@@ -284,7 +358,7 @@ __global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, con
             const int r = tid & (NN - 1); // one x-row per block
             const int rm = (NN - r) & (NN - 1);
             CT* buf = buf_of(NBI + RD);
-            CT* nlr = NL + ((((size_t)(r >> g.lgNS) * (2 * KK) * g.P) + x0) << g.lgNS) + (r & (g.NTs - 1));
+            CT* nlr = NL + ((((size_t)(r >> g.lgNS) * NLN * g.P) + x0) << g.lgNS) + (r & (g.NTs - 1));
             const size_t nls = (size_t)g.P << g.lgNS;
 #pragma unroll
             for (int b = 0; b < 3; b++)
@@ -295,11 +369,11 @@ __global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, con
                 constexpr int r1 = FX::order(2 * q), r2 = FX::order(2 * q + 1);
                 R v1 = (R)0, v2 = (R)0;
                 if constexpr (LONE && q == QL) { // b = 0: phases 0 and 1; b = 1: phase 2
-                    v1 = FX::template row<r1>(vb[2 * b]);
-                    if constexpr (b == 0) v2 = FX::template row<r1>(vb[1]);
+                    v1 = FR::template row<r1>(vb[2 * b], lu, lw);
+                    if constexpr (b == 0) v2 = FR::template row<r1>(vb[1], lu, lw);
                 } else {
-                    if constexpr (r1 >= 0) v1 = FX::template row<r1>(vb[b]);
-                    if constexpr (r2 >= 0) v2 = FX::template row<r2>(vb[b]);
+                    if constexpr (r1 >= 0) v1 = FR::template row<r1>(vb[b], lu, lw);
+                    if constexpr (r2 >= 0) v2 = FR::template row<r2>(vb[b], lu, lw);
                 }
                 buf[(j - J0) * LPZ + lslot<LS>(r)] = CT{v1, v2};
             });
@@ -341,9 +415,9 @@ __global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, con
         const int xl = tid >> LOGNN, r = tid & (NN - 1);
         CT* buf = buf_of(NBI + RD);
         // this thread's element of NL line L is nlr[L * nls] (nidx with the
-        // flux form's 2 KK lines): one base per batch instead of the full
+        // flux form's lines): one base per batch instead of the full
         // index per store
-        CT* nlr = NL + ((((size_t)(r >> g.lgNS) * (2 * KK) * g.P) + (x0 + xl)) << g.lgNS) + (r & (g.NTs - 1));
+        CT* nlr = NL + ((((size_t)(r >> g.lgNS) * NLN * g.P) + (x0 + xl)) << g.lgNS) + (r & (g.NTs - 1));
         const size_t nls = (size_t)g.P << g.lgNS;
         // the base values pass through an empty asm per batch: products shared
         // by rows of different batches are formed again in each batch instead
@@ -359,8 +433,8 @@ __global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, con
 #pragma unroll
             for (int b = 0; b < 3; b++) {
                 R v1 = (R)0, v2 = (R)0;
-                if constexpr (r1 >= 0) v1 = FX::template row<r1>(vb[b]);
-                if constexpr (r2 >= 0) v2 = FX::template row<r2>(vb[b]);
+                if constexpr (r1 >= 0) v1 = FR::template row<r1>(vb[b], lu, lw);
+                if constexpr (r2 >= 0) v2 = FR::template row<r2>(vb[b], lu, lw);
                 buf[((xl * ZP + p) * 3 + b) * LPZ + lslot<LS>(r)] = CT{v1, v2};
             }
         });
