@@ -37,9 +37,15 @@ template <typename CT> __device__ __forceinline__ CT ld_stream(const CT* p)
 
 template <typename CT> __device__ __forceinline__ CT cadd(CT a, CT b) { return CT{a.x + b.x, a.y + b.y}; }
 template <typename CT> __device__ __forceinline__ CT csub(CT a, CT b) { return CT{a.x - b.x, a.y - b.y}; }
+__device__ __forceinline__ double fma_of(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma_of(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+// The fused operations of a product are written out (here and in dft8), so that
+// a transform gives the same bits in every kernel that contains it, whatever
+// each compilation would contract.
 template <typename CT> __device__ __forceinline__ CT cmul(CT a, CT b)
 {
-    return CT{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
+#pragma clang fp contract(off)
+    return CT{fma_of(a.x, b.x, -(a.y * b.y)), fma_of(a.x, b.y, a.y * b.x)};
 }
 template <typename CT> __device__ __forceinline__ CT cconj(CT a) { return CT{a.x, -a.y}; }
 template <typename CT> __device__ __forceinline__ CT cscale(CT a, decltype(a.x) s) { return CT{a.x * s, a.y * s}; }

@@ -80,24 +80,25 @@ template <int SIGN, typename CT> __device__ __forceinline__ void dft4(CT* x) { d
 
 template <int SIGN, typename CT> __device__ __forceinline__ void dft8(CT* x)
 {
+#pragma clang fp contract(off)
     using R = decltype(x[0].x);
     const R h = (R)0.70710678118654752440;
     CT e0 = x[0], e1 = x[2], e2 = x[4], e3 = x[6];
     CT o0 = x[1], o1 = x[3], o2 = x[5], o3 = x[7];
     dft4<SIGN>(e0, e1, e2, e3);
     dft4<SIGN>(o0, o1, o2, o3);
-    // o_s *= exp(SIGN * 2 pi i s / 8)
-    CT w1 = CT{(o1.x - (R)SIGN * o1.y) * h, (o1.y + (R)SIGN * o1.x) * h};
-    CT w2 = cmuli<SIGN>(o2);
-    CT w3 = CT{(-o3.x - (R)SIGN * o3.y) * h, (-o3.y + (R)SIGN * o3.x) * h};
+    // o_s *= exp(SIGN * 2 pi i s / 8); the factor h of s = 1, 3 goes into the sums
+    const CT t1 = CT{o1.x - (R)SIGN * o1.y, o1.y + (R)SIGN * o1.x};
+    const CT t3 = CT{-o3.x - (R)SIGN * o3.y, -o3.y + (R)SIGN * o3.x};
+    const CT w2 = cmuli<SIGN>(o2);
     x[0] = cadd(e0, o0);
     x[4] = csub(e0, o0);
-    x[1] = cadd(e1, w1);
-    x[5] = csub(e1, w1);
+    x[1] = CT{fma_of(t1.x, h, e1.x), fma_of(t1.y, h, e1.y)};
+    x[5] = CT{fma_of(-t1.x, h, e1.x), fma_of(-t1.y, h, e1.y)};
     x[2] = cadd(e2, w2);
     x[6] = csub(e2, w2);
-    x[3] = cadd(e3, w3);
-    x[7] = csub(e3, w3);
+    x[3] = CT{fma_of(t3.x, h, e3.x), fma_of(t3.y, h, e3.y)};
+    x[7] = CT{fma_of(-t3.x, h, e3.x), fma_of(-t3.y, h, e3.y)};
 }
 
 template <int R, int SIGN, typename CT> __device__ __forceinline__ void dftR(CT* x)

@@ -59,6 +59,13 @@ __device__ __forceinline__ double2 xfold_b(double2 X1, double2 X2, double2 w1, d
                    (X1.x * w1.y + X1.y * w1.x) + (X2.y * w2.x - X2.x * w2.y)};
 }
 
+// phase 0 of the same fold
+__device__ __forceinline__ double2 xfold_0(double2 X1, double2 X2)
+{
+#pragma clang fp contract(off)
+    return double2{X1.x + X2.x, X1.y + X2.y};
+}
+
 // var_mpt2spec (program/variables.f90:390-434) for y-mode k at one (m, n):
 // from psi_k (slot k) and phi_k (slot K0-1+k, k >= 1) to u_k, v_k, w_k.
 // At (m,n) = (0,0) the mean-mode rows apply (:418-433) and, when lam is set,
@@ -206,7 +213,8 @@ __global__ __launch_bounds__(XT) void k_xinv(Batch bt, const double2* __restrict
                 X2 = double2{-(X2.y * am1), X2.x * am1};
             }
             CT* bt = buf + (size_t)t * 3 * LP;
-            bt[pidx(r)] = CT{(R)(X1.x + X2.x), (R)(X1.y + X2.y)};
+            const double2 y0 = xfold_0(X1, X2);
+            bt[pidx(r)] = CT{(R)y0.x, (R)y0.y};
 #pragma unroll
             for (int b = 1; b < 3; b++) {
                 const double2 w1 = twP[r * b];
@@ -1128,6 +1136,7 @@ __device__ __forceinline__ void s2m_finish(int k, int mi, int n, double2 u, doub
 __device__ __forceinline__ void dev_term(int li, bool mean, double2 X, double am1, double an1, double ak1, double rak,
                                          double2& psi, double2& phi)
 {
+#pragma clang fp contract(off)
     if (li == DEV_UV) X = double2{-X.y, X.x}; // i uv
     const double a2 = am1 * am1, g2 = an1 * an1;
     double cp, cq;
@@ -1144,13 +1153,36 @@ __device__ __forceinline__ void dev_term(int li, bool mean, double2 X, double am
         cp = am1 * an1 * rak;
         cq = a2;
     }
-    psi.x += cp * X.x;
-    psi.y += cp * X.y;
-    phi.x += cq * X.x;
-    phi.y += cq * X.y;
+    psi.x = __builtin_fma(cp, X.x, psi.x);
+    psi.y = __builtin_fma(cp, X.y, psi.y);
+    phi.x = __builtin_fma(cq, X.x, phi.x);
+    phi.y = __builtin_fma(cq, X.y, phi.y);
     if (mean) {
         if (li == DEV_UV) psi = double2{-(ak1 * X.y), ak1 * X.x}; // -ak uv, X = i uv
         if (li == DEV_F) phi = double2{-(X.y * rak), X.x * rak};
+    }
+}
+
+// Radix-3 unfold of the padded forward x transform, X[m] = sum_b w^{-mb} F_b[m
+// mod MM] at m = r (Xp) and m = r - MM (Xn), tw[j] = exp(2 pi i j/P).  Fused
+// operations are written out here and in dev_term (no contraction), so that the
+// fused x kernels, whose choice depends on the size of a launch, give the same
+// bits.
+template <typename CT>
+__device__ __forceinline__ void xunfold(CT F0, CT F1, CT F2, const double2* __restrict__ tw, int r, int MM, double2& Xp,
+                                        double2& Xn)
+{
+#pragma clang fp contract(off)
+    Xp = Xn = double2{(double)F0.x, (double)F0.y};
+#pragma unroll
+    for (int b = 1; b < 3; b++) {
+        const double fr = (double)(b == 1 ? F1.x : F2.x), fi = (double)(b == 1 ? F1.y : F2.y);
+        const double2 w1 = tw[r * b];        // m = r:      times conj(w1)
+        const double2 w2 = tw[(MM - r) * b]; // m = r - MM: times w2
+        Xp.x = __builtin_fma(fr, w1.x, __builtin_fma(fi, w1.y, Xp.x));
+        Xp.y = __builtin_fma(fi, w1.x, __builtin_fma(-fr, w1.y, Xp.y));
+        Xn.x = __builtin_fma(fr, w2.x, __builtin_fma(-fi, w2.y, Xn.x));
+        Xn.y = __builtin_fma(fi, w2.x, __builtin_fma(fr, w2.y, Xn.y));
     }
 }
 
@@ -1187,12 +1219,8 @@ __device__ __forceinline__ void lhsrhs_k(const Geo& g, int k, int which, bool me
 // precision of the transforms that produced it; the AB2 combination is always
 // evaluated in FP64.  In the mixed form this halves the history's bytes and
 // loses nothing: the stored values carry FP32 transform rounding already.
-__device__ __forceinline__ double2 hist_load(const double2* p) { return *p; }
-__device__ __forceinline__ double2 hist_load(const float2* p)
-{
-    const float2 v = *p;
-    return double2{(double)v.x, (double)v.y};
-}
+template <typename CT> __device__ __forceinline__ double2 hist_wide(CT v) { return double2{(double)v.x, (double)v.y}; }
+template <typename CT> __device__ __forceinline__ double2 hist_load(const CT* p) { return hist_wide(*p); }
 __device__ __forceinline__ void hist_store(double2* p, double2 v, bool stream = false)
 {
     if (stream) st_stream(p, v);
@@ -1280,22 +1308,7 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
             const int n = n0 + t;
             const CT* bt = buf + (size_t)t * 3 * LP;
             double2 Xp, Xn;
-            {
-                const CT F0 = bt[pidx(r)];
-                Xp = double2{(double)F0.x, (double)F0.y};
-                Xn = Xp;
-#pragma unroll
-                for (int b = 1; b < 3; b++) {
-                    const CT Fb = bt[b * LP + pidx(r)];
-                    const double fr = (double)Fb.x, fi = (double)Fb.y;
-                    const double2 w1 = twP[r * b];        // m = r:      times conj(w1)
-                    const double2 w2 = twP[(MM - r) * b]; // m = r - MM: times w2
-                    Xp.x += fr * w1.x + fi * w1.y;
-                    Xp.y += fi * w1.x - fr * w1.y;
-                    Xn.x += fr * w2.x - fi * w2.y;
-                    Xn.y += fi * w2.x + fr * w2.y;
-                }
-            }
+            xunfold(bt[pidx(r)], bt[LP + pidx(r)], bt[2 * LP + pidx(r)], twP, r, MM, Xp, Xn);
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 const double2 X0 = h == 0 ? Xp : Xn;
@@ -1610,19 +1623,9 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
                 const int t = it >> LOGMM, r = it & (MM - 1);
                 const int n = n0 + t;
                 const CT* bt3 = reg + t * 3 * MM;
-                const CT F0 = bt3[pidx(r) ^ xsw<R>(t, 0)];
-                double2 Xp = double2{(double)F0.x, (double)F0.y}, Xn = Xp;
-#pragma unroll
-                for (int b = 1; b < 3; b++) {
-                    const CT Fb = bt3[b * MM + (pidx(r) ^ xsw<R>(t, b))];
-                    const double fr = (double)Fb.x, fi = (double)Fb.y;
-                    const double2 w1 = twPl[r * b];        // m = r:      times conj(w1)
-                    const double2 w2 = twPl[(MM - r) * b]; // m = r - MM: times w2
-                    Xp.x += fr * w1.x + fi * w1.y;
-                    Xp.y += fi * w1.x - fr * w1.y;
-                    Xn.x += fr * w2.x - fi * w2.y;
-                    Xn.y += fi * w2.x + fr * w2.y;
-                }
+                double2 Xp, Xn;
+                xunfold(bt3[pidx(r) ^ xsw<R>(t, 0)], bt3[MM + (pidx(r) ^ xsw<R>(t, 1))],
+                        bt3[2 * MM + (pidx(r) ^ xsw<R>(t, 2))], twPl, r, MM, Xp, Xn);
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     if (h == 1 && r == 0) continue;
@@ -1735,7 +1738,8 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
                 X[h] = val;
             }
             CT* bt3 = reg + t * 3 * MM;
-            bt3[pidx(r) ^ xsw<R>(t, 0)] = CT{(R)(X[0].x + X[1].x), (R)(X[0].y + X[1].y)};
+            const double2 y0 = xfold_0(X[0], X[1]);
+            bt3[pidx(r) ^ xsw<R>(t, 0)] = CT{(R)y0.x, (R)y0.y};
 #pragma unroll
             for (int b = 1; b < 3; b++) {
                 const double2 w1 = twPl[r * b];

@@ -1,6 +1,7 @@
 // plan_x.hip -- launchers of the x kernels for one precision, MWF_R (double
 // or float, set on the compile line).  See plans.hpp.
 #include "kernels.hpp"
+#include "xall.hpp"
 #include "plans.hpp"
 #include "transform.hpp"
 
@@ -56,6 +57,36 @@ static hipError_t launch_xstep(const Batch& bt, int nmem, const Geo& g, hipStrea
     return hipGetLastError();
 }
 
+template <typename R, int LOGMM, int LOGXA>
+static hipError_t launch_xall(const Batch& bt, int nmem, const Geo& g, hipStream_t s, const void* NL, double2* c,
+                              void* onl, void* U, const void* twMM, const double2* twP, int nst, int inv_only)
+{
+    using CT = cplx_t<R>;
+    dim3 grid(g.NN >> (LOGXA - LOGMM), g.K0, nmem);
+    const size_t lds = xa_lds_bytes<R, LOGMM, LOGXA>();
+    if (inv_only)
+        hipLaunchKernelGGL((k_xall<R, LOGMM, LOGXA, true>), grid, dim3(xa_threads<LOGXA>()), lds, s, bt, (const CT*)NL,
+                           c, (CT*)onl, (CT*)U, (const CT*)twMM, twP, nst);
+    else
+        hipLaunchKernelGGL((k_xall<R, LOGMM, LOGXA, false>), grid, dim3(xa_threads<LOGXA>()), lds, s, bt, (const CT*)NL,
+                           c, (CT*)onl, (CT*)U, (const CT*)twMM, twP, nst);
+    return hipGetLastError();
+}
+
+// the fused x kernel of the flux form: k_xall or k_xstep by the size of the launch
+template <typename R, int LOGMM, int LX = 9>
+static hipError_t launch_xf(const Batch& bt, int nmem, const Geo& g, hipStream_t s, const void* NL, double2* c,
+                            void* onl, void* U, const void* twMM, const double2* twP, int nst, int inv_only)
+{
+    if constexpr (LX >= 6 && LX >= LOGMM && LOGMM <= 9) {
+        int lx = xall_log<LOGMM>((g.NN / g.NTx) * g.K0 * nmem);
+        while (lx > LOGMM && (1 << (lx - LOGMM)) > g.NN) lx--; // whole tiles
+        if (lx == LX) return launch_xall<R, LOGMM, LX>(bt, nmem, g, s, NL, c, onl, U, twMM, twP, nst, inv_only);
+        return launch_xf<R, LOGMM, LX - 1>(bt, nmem, g, s, NL, c, onl, U, twMM, twP, nst, inv_only);
+    }
+    return launch_xstep<R, LOGMM, true>(bt, nmem, g, s, NL, c, onl, U, twMM, twP, nst, inv_only);
+}
+
 template <typename R, int LOGMM>
 static hipError_t launch_sxinv(const Geo& g, hipStream_t s, const double2* spec, void* U, const void* twMM,
                                const double2* twP)
@@ -87,7 +118,7 @@ template <typename R> void pick_x(int lm, Plan& p)
         p.xstep = launch_xstep<R, L, false>;    \
         p.xinv_f = launch_xinv<R, L, true>;     \
         p.xfwd_f = launch_xfwd<R, L, true>;     \
-        p.xstep_f = launch_xstep<R, L, true>;   \
+        p.xstep_f = launch_xf<R, L>;   \
         p.sxinv = launch_sxinv<R, L>;           \
         p.sxfwd = launch_sxfwd<R, L>;           \
         break;
@@ -108,6 +139,17 @@ template <typename R> void pick_x(int lm, Plan& p)
     }
 }
 
+template <typename R, int L, int LX = 6> static void prep_xall()
+{
+    if constexpr (LX < 10) {
+        if constexpr (LX >= L) {
+            set_lds(k_xall<R, L, LX, false>, xa_lds_bytes<R, L, LX>());
+            set_lds(k_xall<R, L, LX, true>, xa_lds_bytes<R, L, LX>());
+        }
+        prep_xall<R, L, LX + 1>();
+    }
+}
+
 template <typename R> void prepare_x(int lm)
 {
     switch (lm) {
@@ -121,6 +163,7 @@ template <typename R> void prepare_x(int lm)
         set_lds(k_xfwd<R, L, true>, x_lds<R, L>());             \
         set_lds(k_xstep<R, L, false, true>, xstep_lds<R, L>());  \
         set_lds(k_xstep<R, L, true, true>, xstep_lds<R, L>());   \
+        prep_xall<R, L>();                             \
         set_lds(k_sxinv<R, L>, x_lds<R, L>());         \
         set_lds(k_sxfwd<R, L>, x_lds<R, L>());         \
         break;

@@ -5,6 +5,7 @@
 #include "plans.hpp"
 #include "transform.hpp"
 #include "zflux.hpp"
+#include "zbatch.hpp"
 
 #if !defined(MWF_R) || !defined(MWF_K0)
 #error "compile with -DMWF_R=double|float -DMWF_K0=4|6"
@@ -95,6 +96,21 @@ static hipError_t launch_zc(const Batch& bt, int nmem, const Geo& g, hipStream_t
     return hipGetLastError();
 }
 
+// one batch per row (zbatch.hpp) where it fits, else k_zc with one buffer
+template <typename R, int K0, int LOGNN>
+static hipError_t launch_zs(const Batch& bt, int nmem, const Geo& g, hipStream_t s, const void* U, void* NL,
+                            const void* twNN, const void* twQ)
+{
+    using CT = cplx_t<R>;
+    if constexpr (zs_fits<R, K0, LOGNN>()) {
+        hipLaunchKernelGGL((k_zs<R, K0, LOGNN>), dim3(g.P, 1, nmem), dim3(zs_threads<K0, LOGNN>()),
+                           (zs_lds_bytes<R, K0, LOGNN>()), s, bt, (const CT*)U, (CT*)NL, (const CT*)twNN, (const CT*)twQ);
+        return hipGetLastError();
+    } else {
+        return launch_zc<R, K0, LOGNN, 4>(bt, nmem, g, s, U, NL, twNN, twQ);
+    }
+}
+
 template <typename R, int K0> void pick_z(int ln, Plan& p)
 {
     switch (ln) {
@@ -104,7 +120,8 @@ template <typename R, int K0> void pick_z(int ln, Plan& p)
         p.zf_alt2 = launch_z2<R, K0, L>;        \
         p.zphys = launch_zphys<R, K0, L>;       \
         p.zfwdp = launch_zfwdp<R, L>;           \
-        p.zc = launch_zc<R, K0, L, 4>;          \
+        p.zc = launch_zs<R, K0, L>;             \
+        p.zc_batch = zs_fits<R, K0, L>();       \
         p.zc_alt = launch_zc<R, K0, L, 2>;      \
         break;
         C_(4) C_(5) C_(6) C_(7) C_(8) C_(9)
@@ -136,7 +153,8 @@ template <typename R, int K0> void prepare_z(int ln)
         set_lds(k_z2<R, K0, L>, z2_lds_bytes<R, L>());            \
         set_lds(k_zphys<R, K0, L>, zphys_lds<R, L>());            \
         set_lds(k_zfwd_phys<R, L>, zfp_lds<R, L>());              \
-        set_lds(k_zc<R, K0, L, ZC_ZP, 4, false>, zc_lds_bytes<R, L, ZC_ZP, false>()); \
+        if constexpr (zs_fits<R, K0, L>()) set_lds(k_zs<R, K0, L>, zs_lds_bytes<R, K0, L>()); \
+        else set_lds(k_zc<R, K0, L, ZC_ZP, 4, false>, zc_lds_bytes<R, L, ZC_ZP, false>()); \
         set_lds(k_zc<R, K0, L, ZC_ZP, 2, true>, zc_lds_bytes<R, L, ZC_ZP, true>());   \
         break;
         C_(4) C_(5) C_(6) C_(7) C_(8) C_(9)
