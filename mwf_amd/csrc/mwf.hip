@@ -157,7 +157,7 @@ template <typename T> static int dev_upload(T** d, const T* h, size_t n)
 // ---------------------------------------------------------------------------
 // Autotuner: the role of tra_precompute's FFTW_PATIENT planning
 // (program/transform.fftw5.f90:33-59).  Mode 0 (default): the rule-based plan
-// (k_z for NN <= 512, the fused x kernel wherever it exists).  Mode 1: each
+// (SizeClass::rule).  Mode 1: each
 // new size class times its candidate plans on its own buffers (zero state,
 // best of 3 interleaved rounds of 5 steps) and keeps the fastest; the choice
 // is cached per (precision, K0, MM, NN) for the process, so every handle and
@@ -248,9 +248,16 @@ struct SizeClass {
         HIPCHK(hipStreamSynchronize(st));
         const int mode = g_tune.load();
         if (mode == 1) RCCHK(tune(st));
-        else if (mode >= 2) RCCHK(apply(mode - 2));
+        else RCCHK(apply(mode >= 2 ? mode - 2 : rule()));
         return 0;
     }
+
+    // The rule-based choice: the flux form wherever it exists (M4 steps, advective
+    // and flux: MM = NN = 256 FP64 146 and 97 us, 1024 x 128 modes mixed 84 and 38
+    // us, M6 128^2 FP64 195 and 52 us), with two buffers for rows too long for the
+    // one-batch kernel (NN = 512: FP64 151 and 141 us, FP32 74 and 71 us with one
+    // and two)
+    int rule() const { return !base.zc ? 0 : base.zc_alt && !base.zc_batch ? 8 | 16 : 8; }
 
     // the plan of choice bits ch; the flux form also changes how many lines U
     // and NL hold per x-row, in every member's geometry
