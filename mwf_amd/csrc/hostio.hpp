@@ -1,0 +1,259 @@
+// hostio.hpp -- the host boundary: states, spectra and fields between a
+// caller's arrays and device memory.
+//
+// The reference's (slot, m, n) planes and the device's rows [n][slot][ldM] are
+// transposed on the device (k_planes_out, k_planes_in); the host only copies
+// bytes, through pinned staging chunks that the DMA fills or empties while
+// other chunks are copied by a few threads (a caller's fresh pages fault in on
+// all of them).  A state of M6 2048^2 modes (369 MB) came back in 50 ms when one
+// thread transposed it, and takes 12 ms.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <condition_variable>
+#include <cstring>
+#include <functional>
+#include <memory>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "common.hpp"
+
+constexpr int PLT = 64; // m values per tile
+
+// rows [n][slots][ldM] -> re, im planes (slots, M, NN) column-major
+template <typename CT>
+__global__ __launch_bounds__(256) void k_planes_out(const CT* __restrict__ rows, int slots, int M, int ldM,
+                                                    double* __restrict__ re, double* __restrict__ im)
+{
+    extern __shared__ unsigned char smem_raw[];
+    CT* tile = reinterpret_cast<CT*>(smem_raw); // [slots][PLT + 1]
+    const int m0 = blockIdx.x * PLT, n = blockIdx.y;
+    const int w = M - m0 < PLT ? M - m0 : PLT;
+    for (int i = threadIdx.x; i < slots * PLT; i += blockDim.x) {
+        const int s = i / PLT, m = i % PLT;
+        if (m < w) tile[s * (PLT + 1) + m] = rows[((size_t)n * slots + s) * ldM + m0 + m];
+    }
+    __syncthreads();
+    const size_t o = ((size_t)n * M + m0) * slots;
+    for (int i = threadIdx.x; i < slots * w; i += blockDim.x) {
+        const CT v = tile[(i % slots) * (PLT + 1) + i / slots];
+        re[o + i] = (double)v.x;
+        im[o + i] = (double)v.y;
+    }
+}
+
+// the reverse; the padding m in [M, ldM) of every row is cleared
+template <typename CT>
+__global__ __launch_bounds__(256) void k_planes_in(const double* __restrict__ re, const double* __restrict__ im, int slots,
+                                                   int M, int ldM, CT* __restrict__ rows)
+{
+    using E = decltype(CT{}.x);
+    extern __shared__ unsigned char smem_raw[];
+    CT* tile = reinterpret_cast<CT*>(smem_raw); // [slots][PLT + 1]
+    const int m0 = blockIdx.x * PLT, n = blockIdx.y;
+    const int w = M - m0 < PLT ? M - m0 : PLT, wp = ldM - m0 < PLT ? ldM - m0 : PLT;
+    const size_t o = ((size_t)n * M + m0) * slots;
+    for (int i = threadIdx.x; i < slots * w; i += blockDim.x)
+        tile[(i % slots) * (PLT + 1) + i / slots] = CT{(E)re[o + i], (E)im[o + i]};
+    __syncthreads();
+    for (int i = threadIdx.x; i < slots * PLT; i += blockDim.x) {
+        const int s = i / PLT, m = i % PLT;
+        if (m < wp) rows[((size_t)n * slots + s) * ldM + m0 + m] = m < w ? tile[s * (PLT + 1) + m] : CT{(E)0, (E)0};
+    }
+}
+
+// A few copy threads, shared by every handle of the process and gone with the
+// last one.  run() is one user's at a time; another caller meanwhile does its
+// own work alone.
+class CopyPool {
+public:
+    static std::shared_ptr<CopyPool> get()
+    {
+        static std::mutex mu;
+        static std::weak_ptr<CopyPool> live;
+        std::lock_guard<std::mutex> l(mu);
+        auto p = live.lock();
+        if (!p) live = p = std::shared_ptr<CopyPool>(new CopyPool());
+        return p;
+    }
+    ~CopyPool()
+    {
+        {
+            std::lock_guard<std::mutex> l(mu_);
+            stop_ = true;
+        }
+        cv_.notify_all();
+        for (auto& t : th_) t.join();
+    }
+    // memcpy(dst, src, n) in slices on the pool's threads and the caller's
+    void copy(void* dst, const void* src, size_t n)
+    {
+        constexpr size_t MIN = 128 << 10; // a slice worth a wake-up
+        std::unique_lock<std::mutex> one(user_, std::try_to_lock);
+        if (n < 2 * MIN || !one.owns_lock() || !start()) {
+            std::memcpy(dst, src, n);
+            return;
+        }
+        {
+            std::lock_guard<std::mutex> l(mu_);
+            dst_ = (char*)dst;
+            src_ = (const char*)src;
+            n_ = n;
+            slice_ = std::max(MIN, ((n / (NT + 1) + 4095) / 4096) * 4096);
+            next_ = 0;
+            busy_ = 0;
+            gen_++;
+        }
+        cv_.notify_all();
+        work();
+        std::unique_lock<std::mutex> l(mu_);
+        done_.wait(l, [&] { return busy_ == 0; });
+    }
+
+private:
+    static constexpr int NT = 7;
+    bool start()
+    {
+        if (!th_.empty()) return true;
+        try {
+            for (int i = 0; i < NT; i++) th_.emplace_back([this] { loop(); });
+        } catch (...) { // no more threads: those that started will do
+        }
+        return !th_.empty();
+    }
+    void work()
+    {
+        for (;;) {
+            size_t o, m;
+            {
+                std::lock_guard<std::mutex> l(mu_);
+                if (next_ >= n_) return;
+                o = next_;
+                m = std::min(slice_, n_ - o);
+                next_ += m;
+                busy_++;
+            }
+            std::memcpy(dst_ + o, src_ + o, m);
+            std::lock_guard<std::mutex> l(mu_);
+            if (--busy_ == 0 && next_ >= n_) done_.notify_one();
+        }
+    }
+    void loop()
+    {
+        unsigned long long seen = 0;
+        for (;;) {
+            {
+                std::unique_lock<std::mutex> l(mu_);
+                cv_.wait(l, [&] { return stop_ || gen_ != seen; });
+                if (stop_) return;
+                seen = gen_;
+            }
+            work();
+        }
+    }
+    std::mutex user_, mu_;
+    std::condition_variable cv_, done_;
+    std::vector<std::thread> th_;
+    char* dst_ = nullptr;
+    const char* src_ = nullptr;
+    size_t n_ = 0, slice_ = 0, next_ = 0;
+    int busy_ = 0;
+    unsigned long long gen_ = 0;
+    bool stop_ = false;
+};
+
+// Pinned staging of one handle: chunks, each with the event of its last copy.
+// A transfer that fits one chunk is one copy and one wait (each costs some 20 us
+// whatever its size); longer ones run through all the chunks.
+struct HostStage {
+    static constexpr size_t CHUNK = 4 << 20;
+    static constexpr int NSLOT = 8;
+    char* buf = nullptr;
+    size_t chunk = 0;
+    int nslot = 0;
+    hipEvent_t ev[NSLOT] = {};
+    std::shared_ptr<CopyPool> pool;
+
+    hipError_t init(size_t most) // the largest transfer the handle is likely to make
+    {
+        nslot = most > CHUNK ? NSLOT : 1;
+        chunk = std::min(CHUNK, (most + 4095) / 4096 * 4096);
+        pool = CopyPool::get();
+        hipError_t e = hipHostMalloc((void**)&buf, chunk * nslot, hipHostMallocDefault);
+        for (int i = 0; i < nslot && e == hipSuccess; i++) e = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming);
+        return e;
+    }
+    void release()
+    {
+        for (auto& v : ev)
+            if (v) (void)hipEventDestroy(v);
+        if (buf) (void)hipHostFree(buf);
+        *this = HostStage{};
+    }
+    // device -> host, complete on return; the source's first n0 bytes go to dst0, the rest to dst1
+    hipError_t d2h(hipStream_t st, const void* src, size_t bytes, void* dst0, size_t n0, void* dst1)
+    {
+        const size_t nc = (bytes + chunk - 1) / chunk;
+        auto len = [&](size_t c) { return std::min(chunk, bytes - c * chunk); };
+        auto slot = [&](size_t c) { return buf + (c % nslot) * chunk; };
+        auto issue = [&](size_t c) {
+            hipError_t e = hipMemcpyAsync(slot(c), (const char*)src + c * chunk, len(c), hipMemcpyDeviceToHost, st);
+            return e != hipSuccess || nc == 1 ? e : hipEventRecord(ev[c % nslot], st);
+        };
+        hipError_t e = hipSuccess;
+        for (size_t c = 0; c < nc && c < (size_t)nslot && e == hipSuccess; c++) e = issue(c);
+        for (size_t c = 0; c < nc && e == hipSuccess; c++) {
+            if ((e = nc == 1 ? hipStreamSynchronize(st) : hipEventSynchronize(ev[c % nslot])) != hipSuccess) break;
+            const size_t a = c * chunk, b = a + len(c), m = std::min(std::max(a, n0), b);
+            if (m > a) pool->copy((char*)dst0 + a, slot(c), m - a);
+            if (b > m) pool->copy((char*)dst1 + (m - n0), slot(c) + (m - a), b - m);
+            if (c + nslot < nc) e = issue(c + nslot);
+        }
+        if (e != hipSuccess) (void)hipStreamSynchronize(st); // nothing may still write the chunks
+        return e;
+    }
+    hipError_t d2h(hipStream_t st, void* dst, const void* src, size_t bytes) { return d2h(st, src, bytes, dst, bytes, nullptr); }
+    // host -> device, the sources read on return; n0 bytes from src0, the rest from src1
+    hipError_t h2d(hipStream_t st, void* dst, size_t bytes, const void* src0, size_t n0, const void* src1)
+    {
+        const size_t nc = (bytes + chunk - 1) / chunk;
+        hipError_t e = hipSuccess;
+        for (size_t c = 0; c < nc && e == hipSuccess; c++) {
+            char* s = buf + (c % nslot) * chunk;
+            const size_t a = c * chunk, b = std::min(a + chunk, bytes), m = std::min(std::max(a, n0), b);
+            if (c >= (size_t)nslot && (e = hipEventSynchronize(ev[c % nslot])) != hipSuccess) break;
+            if (m > a) pool->copy(s, (const char*)src0 + a, m - a);
+            if (b > m) pool->copy(s + (m - a), (const char*)src1 + (m - n0), b - m);
+            if ((e = hipMemcpyAsync((char*)dst + a, s, b - a, hipMemcpyHostToDevice, st)) != hipSuccess) break;
+            if (nc > 1) e = hipEventRecord(ev[c % nslot], st);
+        }
+        const hipError_t w = hipStreamSynchronize(st); // the chunks are free for the next transfer
+        return e != hipSuccess ? e : w;
+    }
+    hipError_t h2d(hipStream_t st, void* dst, const void* src, size_t bytes) { return h2d(st, dst, bytes, src, bytes, nullptr); }
+};
+
+// Planes of `slots` slots, both directions; scratch holds 2 NN M slots doubles.
+template <typename CT>
+inline hipError_t planes_d2h(HostStage& hs, hipStream_t st, const Geo& g, int slots, const CT* rows, double* scratch,
+                             double* re, double* im)
+{
+    const size_t n = (size_t)g.NN * g.M * slots;
+    hipLaunchKernelGGL(k_planes_out<CT>, dim3((g.M + PLT - 1) / PLT, g.NN), dim3(256), slots * (PLT + 1) * sizeof(CT), st,
+                       rows, slots, g.M, g.ldM, scratch, scratch + n);
+    hipError_t e = hipGetLastError();
+    return e != hipSuccess ? e : hs.d2h(st, scratch, 2 * sizeof(double) * n, re, sizeof(double) * n, im);
+}
+template <typename CT>
+inline hipError_t planes_h2d(HostStage& hs, hipStream_t st, const Geo& g, int slots, const double* re, const double* im,
+                             double* scratch, CT* rows)
+{
+    const size_t n = (size_t)g.NN * g.M * slots;
+    const hipError_t e = hs.h2d(st, scratch, 2 * sizeof(double) * n, re, sizeof(double) * n, im);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_planes_in<CT>, dim3((g.ldM + PLT - 1) / PLT, g.NN), dim3(256), slots * (PLT + 1) * sizeof(CT), st,
+                       scratch, scratch + n, slots, g.M, g.ldM, rows);
+    return hipGetLastError();
+}

@@ -1279,7 +1279,11 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
     // u_k until w_k arrives, phi[] holds v_k (am2+an2) until then
     double2 psi[IPT][2] = {}, phi[IPT][2] = {};
 
+#pragma unroll 1
     for (int li = 0; li < (FLUX ? 4 : 3); li++) {
+        // opaque copy of the thread index: keeps item arithmetic inside the loop
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
         if (k == 0 && (FLUX ? li > DEV_F : li == 1)) continue;
         const int slot = FLUX ? dev_line(k) + li : (li == 0 ? k : (li == 1 ? g.K0 - 1 + k : 2 * g.K0 - 1 + k));
         const CT* pan = nl_panel(g, NL, n0, slot);
@@ -1299,7 +1303,7 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
             buf[((size_t)t * 3 + b) * LP + pidx(a)] = v;
         }
         __syncthreads();
-        ip_fft<CT, LOGMM, -1, XT, 3 * (XTILE >> LOGMM)>(buf, 3 * NT, twMM);
+        ip_fft<CT, LOGMM, -1, XT, 3 * (XTILE >> LOGMM)>(buf, 3 * NT, twMM, tid);
 #pragma unroll
         for (int q = 0; q < IPT; q++) {
             const int it = tid + q * XT;

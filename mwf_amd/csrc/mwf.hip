@@ -24,6 +24,7 @@
 
 #include "../../include/mwf.h"
 #include "diag.hpp"
+#include "hostio.hpp"
 #include "plans.hpp"
 
 static thread_local std::string g_err;
@@ -413,41 +414,6 @@ struct SizeClass {
     }
 };
 
-// reference mpt / spec (re, im planes, (slots, M, NN) column-major) <-> device
-// rows [NN][slots][ldM]
-static void to_dev_rows(const Geo& g, int slots, size_t elems, const double* re, const double* im, double2* d)
-{
-    std::memset(d, 0, sizeof(double2) * elems);
-    for (int n = 0; n < g.NN; n++)
-        for (int m = 0; m < g.M; m++)
-            for (int k = 0; k < slots; k++) {
-                const size_t i = (size_t)k + (size_t)slots * ((size_t)m + (size_t)g.M * n);
-                d[((size_t)n * slots + k) * g.ldM + m] = double2{re[i], im[i]};
-            }
-}
-
-static void from_dev_rows(const Geo& g, int slots, const double2* d, double* re, double* im)
-{
-    for (int n = 0; n < g.NN; n++)
-        for (int m = 0; m < g.M; m++)
-            for (int k = 0; k < slots; k++) {
-                const size_t i = (size_t)k + (size_t)slots * ((size_t)m + (size_t)g.M * n);
-                const double2 v = d[((size_t)n * slots + k) * g.ldM + m];
-                re[i] = v.x;
-                im[i] = v.y;
-            }
-}
-
-static void to_dev_layout(const Geo& g, size_t elems, const double* re, const double* im, double2* d)
-{
-    to_dev_rows(g, g.K, elems, re, im, d);
-}
-
-static void from_dev_layout(const Geo& g, const double2* d, double* re, double* im)
-{
-    from_dev_rows(g, g.K, d, re, im);
-}
-
 // ---------------------------------------------------------------------------
 // profiling
 // ---------------------------------------------------------------------------
@@ -558,9 +524,8 @@ struct mwf_handle {
     size_t phys_elems = 0;
     void* diag = nullptr;      // device scratch of the diagnostics
     size_t diag_bytes = 0;
-    double2* hstage = nullptr; // pinned host staging, one device mpt
+    HostStage hs;              // pinned staging of host transfers
     double2* tspec = nullptr;  // device spec of the transform entry points
-    double2* hspec = nullptr;  // pinned host staging of one spec
     Profiler prof;
 };
 
@@ -572,9 +537,8 @@ static void destroy(mwf_handle* h)
     h->cls.reset();
     if (h->phys) (void)hipFree(h->phys);
     if (h->diag) (void)hipFree(h->diag);
-    if (h->hstage) (void)hipHostFree(h->hstage);
+    h->hs.release();
     if (h->tspec) (void)hipFree(h->tspec);
-    if (h->hspec) (void)hipHostFree(h->hspec);
     if (h->st) (void)hipStreamDestroy(h->st);
     delete h;
 }
@@ -592,7 +556,7 @@ extern "C" int mwf_create(const mwf_params* p, mwf_handle** out)
         h->cls.reset(new SizeClass());
         rc = h->cls->init({*p}, h->st);
     }
-    if (!rc && hipHostMalloc((void**)&h->hstage, sizeof(double2) * h->cls->mpt_elems, hipHostMallocDefault) != hipSuccess)
+    if (!rc && h->hs.init(sizeof(double) * h->cls->g0.KK * h->cls->g0.P * h->cls->g0.Q) != hipSuccess)
         rc = fail(MWF_E_NOMEM, "hipHostMalloc failed");
     if (rc) {
         destroy(h);
@@ -608,21 +572,21 @@ extern "C" int mwf_destroy(mwf_handle* h)
     return 0;
 }
 
+// host mpt planes to and from device rows; the planes lie in scratch on the
+// device (2 NN M K doubles: the scratch mpt cs, or U where cs is the rows)
 static int upload_mpt(mwf_handle* h, const double* re, const double* im, double2* dst)
 {
     SizeClass& k = *h->cls;
-    to_dev_layout(k.g0, k.mpt_elems, re, im, h->hstage);
-    HIPCHK(hipMemcpyAsync(dst, h->hstage, sizeof(double2) * k.mpt_elems, hipMemcpyHostToDevice, h->st));
-    HIPCHK(hipStreamSynchronize(h->st));
+    double* scratch = static_cast<double*>(dst == k.cs ? k.U : (void*)k.cs);
+    HIPCHK(planes_h2d(h->hs, h->st, k.g0, k.g0.K, re, im, scratch, dst));
     return 0;
 }
 
 static int download_mpt(mwf_handle* h, const double2* src, double* re, double* im)
 {
     SizeClass& k = *h->cls;
-    HIPCHK(hipMemcpyAsync(h->hstage, src, sizeof(double2) * k.mpt_elems, hipMemcpyDeviceToHost, h->st));
-    HIPCHK(hipStreamSynchronize(h->st));
-    from_dev_layout(k.g0, h->hstage, re, im);
+    double* scratch = static_cast<double*>(src == k.cs ? k.U : (void*)k.cs);
+    HIPCHK(planes_d2h(h->hs, h->st, k.g0, k.g0.K, src, scratch, re, im));
     return 0;
 }
 
@@ -753,10 +717,10 @@ extern "C" int mwf_mpt2phys(mwf_handle* h, const double* re, const double* im, d
     if (!h || !re || !im || !phys) return fail(MWF_E_ARG, "null argument");
     SizeClass& k = *h->cls;
     const Geo& g = k.g0;
+    k.u_valid = false; // U is overwritten
     RCCHK(upload_mpt(h, re, im, k.cs));
     RCCHK(phys_of(h, k.cs));
-    HIPCHK(hipMemcpyAsync(phys, h->phys, sizeof(double) * g.KK * g.Q * g.P, hipMemcpyDeviceToHost, h->st));
-    HIPCHK(hipStreamSynchronize(h->st));
+    HIPCHK(h->hs.d2h(h->st, phys, h->phys, sizeof(double) * g.KK * g.Q * g.P));
     return 0;
 }
 
@@ -765,8 +729,6 @@ static int ensure_tspec(mwf_handle* h)
     const Geo& g = h->cls->g0;
     const size_t n = (size_t)g.NN * g.KK * g.ldM;
     if (!h->tspec) HIPCHK(hipMalloc((void**)&h->tspec, sizeof(double2) * n));
-    if (!h->hspec && hipHostMalloc((void**)&h->hspec, sizeof(double2) * n, hipHostMallocDefault) != hipSuccess)
-        return fail(MWF_E_NOMEM, "hipHostMalloc failed");
     return 0;
 }
 
@@ -777,15 +739,12 @@ extern "C" int mwf_spec2phys(mwf_handle* h, const double* re, const double* im, 
     const Geo& g = k.g0;
     RCCHK(ensure_tspec(h));
     RCCHK(ensure_phys(h));
-    const size_t n = (size_t)g.NN * g.KK * g.ldM;
-    to_dev_rows(g, g.KK, n, re, im, h->hspec);
-    HIPCHK(hipMemcpyAsync(h->tspec, h->hspec, sizeof(double2) * n, hipMemcpyHostToDevice, h->st));
-    k.u_valid = false; // U is overwritten
+    k.u_valid = false; // U is overwritten, first by the planes
+    HIPCHK(planes_h2d(h->hs, h->st, g, g.KK, re, im, static_cast<double*>(k.U), h->tspec));
     hipError_t e = k.plan.sxinv(g, h->st, h->tspec, k.U, k.twMM(), k.twPd);
     if (e == hipSuccess) e = k.plan.zphys(k.bt, 1, g, h->st, k.U, h->phys, k.twNN(), k.twQ());
     if (e != hipSuccess) return fail(MWF_E_HIP, hipGetErrorString(e));
-    HIPCHK(hipMemcpyAsync(phys, h->phys, sizeof(double) * g.KK * g.Q * g.P, hipMemcpyDeviceToHost, h->st));
-    HIPCHK(hipStreamSynchronize(h->st));
+    HIPCHK(h->hs.d2h(h->st, phys, h->phys, sizeof(double) * g.KK * g.Q * g.P));
     return 0;
 }
 
@@ -796,14 +755,12 @@ extern "C" int mwf_phys2spec(mwf_handle* h, const double* phys, double* re, doub
     const Geo& g = k.g0;
     RCCHK(ensure_tspec(h));
     RCCHK(ensure_phys(h));
-    const size_t n = (size_t)g.NN * g.KK * g.ldM;
-    HIPCHK(hipMemcpyAsync(h->phys, phys, sizeof(double) * g.KK * g.Q * g.P, hipMemcpyHostToDevice, h->st));
+    HIPCHK(h->hs.h2d(h->st, h->phys, phys, sizeof(double) * g.KK * g.Q * g.P));
     hipError_t e = k.plan.zfwdp(g, h->st, h->phys, k.NL, k.twNN(), k.twQ());
     if (e == hipSuccess) e = k.plan.sxfwd(g, h->st, k.NL, h->tspec, k.twMM(), k.twPd);
     if (e != hipSuccess) return fail(MWF_E_HIP, hipGetErrorString(e));
-    HIPCHK(hipMemcpyAsync(h->hspec, h->tspec, sizeof(double2) * n, hipMemcpyDeviceToHost, h->st));
-    HIPCHK(hipStreamSynchronize(h->st));
-    from_dev_rows(g, g.KK, h->hspec, re, im);
+    // the field has been read: its buffer takes the planes
+    HIPCHK(planes_d2h(h->hs, h->st, g, g.KK, h->tspec, h->phys, re, im));
     return 0;
 }
 
@@ -815,11 +772,7 @@ extern "C" int mwf_get_onl(mwf_handle* h, double* re, double* im, int32_t* first
     SizeClass& k = *h->cls;
     *first_step = k.nst;
     if (k.hsz == sizeof(double2)) return download_mpt(h, static_cast<double2*>(k.onl), re, im);
-    float2* f = reinterpret_cast<float2*>(h->hstage);
-    HIPCHK(hipMemcpyAsync(f, k.onl, sizeof(float2) * k.mpt_elems, hipMemcpyDeviceToHost, h->st));
-    HIPCHK(hipStreamSynchronize(h->st));
-    for (size_t i = k.mpt_elems; i-- > 0;) h->hstage[i] = double2{(double)f[i].x, (double)f[i].y};
-    from_dev_layout(k.g0, h->hstage, re, im);
+    HIPCHK(planes_d2h(h->hs, h->st, k.g0, k.g0.K, static_cast<const float2*>(k.onl), reinterpret_cast<double*>(k.cs), re, im));
     return 0;
 }
 
@@ -830,11 +783,7 @@ extern "C" int mwf_set_onl(mwf_handle* h, const double* re, const double* im)
     if (k.hsz == sizeof(double2)) {
         RCCHK(upload_mpt(h, re, im, static_cast<double2*>(k.onl)));
     } else {
-        to_dev_layout(k.g0, k.mpt_elems, re, im, h->hstage);
-        float2* f = reinterpret_cast<float2*>(h->hstage);
-        for (size_t i = 0; i < k.mpt_elems; i++) f[i] = float2{(float)h->hstage[i].x, (float)h->hstage[i].y};
-        HIPCHK(hipMemcpyAsync(k.onl, f, sizeof(float2) * k.mpt_elems, hipMemcpyHostToDevice, h->st));
-        HIPCHK(hipStreamSynchronize(h->st));
+        HIPCHK(planes_h2d(h->hs, h->st, k.g0, k.g0.K, re, im, reinterpret_cast<double*>(k.cs), static_cast<float2*>(k.onl)));
     }
     k.nst = 0;
     return 0;
@@ -1075,8 +1024,7 @@ struct mwf_ens {
     std::vector<ClassTrack> trk;            // per class
     std::vector<std::pair<int, int>> where; // member -> (class, index in class)
     std::vector<mwf_params> params;
-    double2* hstage = nullptr;
-    size_t hstage_elems = 0;
+    HostStage hs;           // pinned staging of host transfers
     double* ebuf = nullptr; // host, one energy per member
     // step graphs by (steps, sample at the end), built on demand
     std::map<std::pair<int, int>, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
@@ -1118,7 +1066,7 @@ static void ens_destroy(mwf_ens* e)
     for (auto v : e->cev)
         if (v) (void)hipEventDestroy(v);
     if (e->fork) (void)hipEventDestroy(e->fork);
-    if (e->hstage) (void)hipHostFree(e->hstage);
+    e->hs.release();
     delete[] e->ebuf;
     if (e->st) (void)hipStreamDestroy(e->st);
     delete e;
@@ -1163,9 +1111,7 @@ extern "C" int mwf_ens_create(const mwf_params* members, int32_t n, mwf_ens** ou
         maxel = std::max(maxel, k->mpt_elems);
         e->classes.push_back(std::move(k));
     }
-    if (!rc && hipHostMalloc((void**)&e->hstage, sizeof(double2) * maxel, hipHostMallocDefault) != hipSuccess)
-        rc = fail(MWF_E_NOMEM, "hipHostMalloc failed");
-    e->hstage_elems = maxel;
+    if (!rc && e->hs.init(sizeof(double2) * maxel) != hipSuccess) rc = fail(MWF_E_NOMEM, "hipHostMalloc failed");
     if (rc) {
         ens_destroy(e);
         return rc;
@@ -1184,10 +1130,8 @@ extern "C" int mwf_ens_set_state(mwf_ens* e, int32_t member, const double* re, c
 {
     if (!e || !re || !im || member < 0 || member >= (int)e->where.size()) return fail(MWF_E_ARG, "bad arguments");
     SizeClass& k = *e->classes[e->where[member].first];
-    to_dev_layout(k.g0, k.mpt_elems, re, im, e->hstage);
-    HIPCHK(hipMemcpyAsync(k.c + k.mpt_elems * e->where[member].second, e->hstage, sizeof(double2) * k.mpt_elems,
-                          hipMemcpyHostToDevice, e->st));
-    HIPCHK(hipStreamSynchronize(e->st));
+    HIPCHK(planes_h2d(e->hs, e->st, k.g0, k.g0.K, re, im, reinterpret_cast<double*>(k.cs),
+                      k.c + k.mpt_elems * e->where[member].second));
     // AB2 restarts with forward Euler for the whole ensemble (vel_precompute's nst)
     for (auto& c : e->classes) {
         c->nst = 1;
@@ -1201,10 +1145,8 @@ extern "C" int mwf_ens_get_state(mwf_ens* e, int32_t member, double* re, double*
 {
     if (!e || !re || !im || member < 0 || member >= (int)e->where.size()) return fail(MWF_E_ARG, "bad arguments");
     SizeClass& k = *e->classes[e->where[member].first];
-    HIPCHK(hipMemcpyAsync(e->hstage, k.c + k.mpt_elems * e->where[member].second, sizeof(double2) * k.mpt_elems,
-                          hipMemcpyDeviceToHost, e->st));
-    HIPCHK(hipStreamSynchronize(e->st));
-    from_dev_layout(k.g0, e->hstage, re, im);
+    HIPCHK(planes_d2h(e->hs, e->st, k.g0, k.g0.K, static_cast<const double2*>(k.c) + k.mpt_elems * e->where[member].second,
+                      reinterpret_cast<double*>(k.cs), re, im));
     return 0;
 }
 
@@ -1302,10 +1244,11 @@ static int ens_graph(mwf_ens* e, int steps, bool sample, hipGraphExec_t* exec)
     return 0;
 }
 
-// Move the device trace buffers to the host vectors and empty them.
+// Move the device trace buffers to the host vectors and empty them (reading
+// every member's traces drains once, not once per member).
 static int ens_drain(mwf_ens* e)
 {
-    if (e->track_every <= 0) return 0;
+    if (e->track_every <= 0 || e->pending == 0) return 0;
     HIPCHK(hipStreamSynchronize(e->st));
     std::vector<double> eb, fb;
     std::vector<long long> rl;
