@@ -79,7 +79,7 @@ struct Geo {
     int NTs;           // z-modes per NL piece (a multiple of NTx, power of two)
     int lgNS;          // log2(NTs)
     int XB;            // x-rows per z-kernel block
-    int UL, NLL;       // lines per x-row of U and NL: 2 KK and KK (advective form), KK and 4 K0 - 2 (flux form)
+    int UL, NLL;       // lines per x-row of U and NL: 2 KK and KK (advective form), KK and 4 K0 - 2 or 5 K0 - 3 (flux form)
     double alpha, gamma, re, dt, drag, vdrag, hypo, cth, sth, beta;
     double scale;      // 1/(P*Q), transform.fftw5.f90:242
     int dragall;
@@ -144,3 +144,6 @@ __device__ __forceinline__ double ak2_of(int k, double beta) { return -k * k * b
 enum { DEV_UW, DEV_F, DEV_UV, DEV_E };
 __host__ __device__ constexpr int dev_line(int k) { return k == 0 ? 0 : 4 * k - 2; }
 __host__ __device__ constexpr int dev_lines(int K0) { return 4 * K0 - 2; }
+// with the vw share of E_k on a line of its own, dev_lines + k - 1 (FP64 rows of
+// 1024 points; Geo::NLL tells the x kernels)
+__host__ __device__ constexpr int dev_lines_split(int K0) { return 5 * K0 - 3; }

@@ -1287,6 +1287,7 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
         if (k == 0 && (FLUX ? li > DEV_F : li == 1)) continue;
         const int slot = FLUX ? dev_line(k) + li : (li == 0 ? k : (li == 1 ? g.K0 - 1 + k : 2 * g.K0 - 1 + k));
         const CT* pan = nl_panel(g, NL, n0, slot);
+        const ptrdiff_t evw = (ptrdiff_t)(dev_lines(g.K0) + k - 1 - slot) * g.P * g.NTs;
         // load NL rows, decimated by b = x mod 3
 #pragma unroll
         for (int q = 0; q < 3 * IPT; q++) {
@@ -1296,7 +1297,9 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
             const int a = x / 3, b = x - 3 * a;
             const int po = pan_at(g, it);
             CT v = pan[po];
-            if (bt.nl_part) { // the z pass's three fold-phase partials: ((P0 + P1) + P2) / (PQ)
+            if (FLUX && li == DEV_E && g.NLL > dev_lines(g.K0)) // the vw share of E
+                v = cadd(v, pan[po + evw]);
+            if (!FLUX && bt.nl_part) { // the z pass's three fold-phase partials: ((P0 + P1) + P2) / (PQ)
                 const CT v1 = pan[po + bt.nl_part], v2 = pan[po + 2 * bt.nl_part];
                 v = cscale(cadd(cadd(v, v1), v2), (R)g.scale);
             }
@@ -1568,9 +1571,13 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
                 const CT* pan = panel_of(li);
                 // NL element, or the sum ((P0 + P1) + P2) / (PQ) of the three
                 // fold-phase partials of the phase-split z kernel
-                const size_t nlp = bt.nl_part;
+                const size_t nlp = FLUX ? 0 : bt.nl_part;
+                // flux form: where E's vw share has a line of its own, add it
+                const bool esum = FLUX && li == DEV_E && g.NLL > dev_lines(g.K0);
+                const ptrdiff_t evw = (ptrdiff_t)(dev_lines(g.K0) + k - 1 - (dev_line(k) + DEV_E)) * g.P * g.NTs;
                 auto nl_at = [&](const CT* p) {
                     CT v = ld_stream(p);
+                    if (FLUX && esum) v = cadd(v, ld_stream(p + evw));
                     if (nlp) v = cscale(cadd(cadd(v, ld_stream(p + nlp)), ld_stream(p + 2 * nlp)), (R)g.scale);
                     return v;
                 };

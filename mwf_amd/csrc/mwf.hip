@@ -221,8 +221,9 @@ struct SizeClass {
             return fail(MWF_E_ARG, "no kernel for this size");
         const size_t rsz = prec == MWF_MIXED ? sizeof(float2) : sizeof(double2);
         mpt_elems = (size_t)g0.NN * g0.K * g0.ldM;
-        // room for either form: U holds up to 2 KK lines per x-row, NL dev_lines(K0) >= KK
-        const size_t u_el = (size_t)g0.P * 2 * g0.KK * g0.NN, nl_el = (size_t)g0.P * dev_lines(g0.K0) * g0.NN;
+        // room for either form: U holds up to 2 KK lines per x-row, NL those of the flux form, at least KK
+        const int nll = base.zc_split ? dev_lines_split(g0.K0) : dev_lines(g0.K0);
+        const size_t u_el = (size_t)g0.P * 2 * g0.KK * g0.NN, nl_el = (size_t)g0.P * nll * g0.NN;
         nepart = (g0.NN / g0.NTx) * g0.K0;
         RCCHK(dev_upload(&geos, geos_h.data(), geos_h.size()));
         HIPCHK(hipMalloc((void**)&c, sizeof(double2) * mpt_elems * nmem));
@@ -253,12 +254,17 @@ struct SizeClass {
         return 0;
     }
 
-    // The rule-based choice: the flux form wherever it exists (M4 steps, advective
-    // and flux: MM = NN = 256 FP64 146 and 97 us, 1024 x 128 modes mixed 84 and 38
-    // us, M6 128^2 FP64 195 and 52 us), with two buffers for rows too long for the
-    // one-batch kernel (NN = 512: FP64 151 and 141 us, FP32 74 and 71 us with one
-    // and two)
-    int rule() const { return !base.zc ? 0 : base.zc_alt && !base.zc_batch ? 8 | 16 : 8; }
+    // The rule-based choice: the flux form (M4 steps, advective and flux: MM = NN
+    // = 256 FP64 146 and 97 us, 1024 x 128 modes mixed 84 and 38 us; M6 2048^2
+    // FP64 5140 and 3140 us), its z kernel with two buffers for rows too long for
+    // the one-batch kernel (NN = 512: FP64 151 and 141 us with one and two, FP32 74
+    // and 71) and for many rows of 256 points (MM = 256, 1024, one batch and two
+    // buffers: FP64 M4 44 and 52, 161 and 148; FP32 M6 41 and 43, 157 and 117).
+    int rule() const
+    {
+        if (!base.zc) return 0;
+        return base.zc_alt && (!base.zc_batch || (g0.NN == 256 && g0.MM >= 512)) ? 8 | 16 : 8;
+    }
 
     // the plan of choice bits ch; the flux form also changes how many lines U
     // and NL hold per x-row, in every member's geometry
@@ -284,7 +290,7 @@ struct SizeClass {
         // panels into LDS and takes them with the split x kernels
         if ((ch & 2) || (ph3 && prec == MWF_MIXED)) plan.xstep = nullptr;
         bt.nl_part = ph3 ? bt.nl_stride * nmem : 0;
-        const int UL = flux ? g0.KK : 2 * g0.KK, NLL = flux ? dev_lines(g0.K0) : g0.KK;
+        const int UL = flux ? g0.KK : 2 * g0.KK, NLL = !flux ? g0.KK : base.zc_split ? dev_lines_split(g0.K0) : dev_lines(g0.K0);
         if (g0.UL != UL) {
             g0.UL = UL;
             g0.NLL = NLL;

@@ -80,9 +80,10 @@ static hipError_t launch_zfwdp(const Geo& g, hipStream_t s, const double* phys, 
 
 // flux-form z kernel: two pairs per batch
 constexpr int ZC_ZP = 2;
-// W: waves per SIMD the kernel is compiled for: 4 (two 512-thread blocks per
-// CU, 128 VGPRs, transforms in place) or 2 (one block, 256 VGPRs, ping-pong
-// transforms)
+// W: 4 (two 512-thread blocks per CU, 128 VGPRs, one transform buffer) or 2
+// (two buffers; in FP64 one block per CU with 256 VGPRs, in FP32 two blocks
+// still: M6 NN = 512, 149 us with one, 117 with two)
+template <typename R, int W> constexpr int zc_waves() { return sizeof(R) == 4 ? 4 : W; }
 template <typename R, int K0, int LOGNN, int W>
 static hipError_t launch_zc(const Batch& bt, int nmem, const Geo& g, hipStream_t s, const void* U, void* NL,
                             const void* twNN, const void* twQ)
@@ -90,8 +91,21 @@ static hipError_t launch_zc(const Batch& bt, int nmem, const Geo& g, hipStream_t
     using CT = cplx_t<R>;
     constexpr int XB = zc_threads<LOGNN>() >> LOGNN;
     dim3 grid((g.P + XB - 1) / XB, 1, nmem);
-    hipLaunchKernelGGL((k_zc<R, K0, LOGNN, ZC_ZP, W, W == 2>), grid, dim3(zc_threads<LOGNN>()),
+    hipLaunchKernelGGL((k_zc<R, K0, LOGNN, ZC_ZP, zc_waves<R, W>(), W == 2>), grid, dim3(zc_threads<LOGNN>()),
                        (zc_lds_bytes<R, LOGNN, ZC_ZP, W == 2>()), s, bt, (const CT*)U, (CT*)NL, (const CT*)twNN,
+                       (const CT*)twQ);
+    return hipGetLastError();
+}
+
+template <typename R, int K0, int LOGNN>
+static hipError_t launch_zc3(const Batch& bt, int nmem, const Geo& g, hipStream_t s, const void* U, void* NL,
+                             const void* twNN, const void* twQ)
+{
+    using CT = cplx_t<R>;
+    static_assert(zc_threads<LOGNN>() == (1 << LOGNN), "one x-row per block");
+    if (g.P % 8) return hipErrorInvalidValue; // the XCD mapping needs whole rounds of 8
+    hipLaunchKernelGGL((k_zc3<R, K0, LOGNN, ZC_ZP>), dim3(3 * g.P, 1, nmem), dim3(zc_threads<LOGNN>()),
+                       (zc_lds_bytes<R, LOGNN, ZC_ZP, false>()), s, bt, (const CT*)U, (CT*)NL, (const CT*)twNN,
                        (const CT*)twQ);
     return hipGetLastError();
 }
@@ -137,8 +151,13 @@ template <typename R, int K0> void pick_z(int ln, Plan& p)
         p.zphys = launch_zphys<R, K0, 10>;
         p.zfwdp = launch_zfwdp<R, 10>;
         // the flux z kernel holds all three phases of a 3072-point row at
-        // 1024 threads (4 waves per SIMD) in FP32 only
+        // 1024 threads (4 waves per SIMD) in FP32 only; in FP64 three blocks
+        // share the row
         if constexpr (std::is_same<R, float>::value) p.zc = launch_zc<R, K0, 10, 4>;
+        else {
+            p.zc = launch_zc3<R, K0, 10>;
+            p.zc_split = true;
+        }
         break;
     default: break;
     }
@@ -155,7 +174,7 @@ template <typename R, int K0> void prepare_z(int ln)
         set_lds(k_zfwd_phys<R, L>, zfp_lds<R, L>());              \
         if constexpr (zs_fits<R, K0, L>()) set_lds(k_zs<R, K0, L>, zs_lds_bytes<R, K0, L>()); \
         else set_lds(k_zc<R, K0, L, ZC_ZP, 4, false>, zc_lds_bytes<R, L, ZC_ZP, false>()); \
-        set_lds(k_zc<R, K0, L, ZC_ZP, 2, true>, zc_lds_bytes<R, L, ZC_ZP, true>());   \
+        set_lds(k_zc<R, K0, L, ZC_ZP, zc_waves<R, 2>(), true>, zc_lds_bytes<R, L, ZC_ZP, true>());   \
         break;
         C_(4) C_(5) C_(6) C_(7) C_(8) C_(9)
 #undef C_
@@ -171,6 +190,7 @@ template <typename R, int K0> void prepare_z(int ln)
         set_lds(k_zfwd_phys<R, 10>, zfp_lds<R, 10>());
         if constexpr (std::is_same<R, float>::value)
             set_lds(k_zc<R, K0, 10, ZC_ZP, 4, false>, zc_lds_bytes<R, 10, ZC_ZP, false>());
+        else set_lds(k_zc3<R, K0, 10, ZC_ZP>, zc_lds_bytes<R, 10, ZC_ZP, false>());
         break;
     default: break;
     }

@@ -37,6 +37,7 @@ struct Plan {
     hipError_t (*zc)(const Batch&, int, const Geo&, hipStream_t, const void*, void*, const void*, const void*) = nullptr;
     hipError_t (*zc_alt)(const Batch&, int, const Geo&, hipStream_t, const void*, void*, const void*,
                          const void*) = nullptr; // the flux z kernel at 2 waves per SIMD instead of 4
+    bool zc_split = false; // zc writes dev_lines_split(K0) lines
     bool zc_batch = false; // zc takes a whole x-row in one batch (zbatch.hpp)
     hipError_t (*xinv_f)(const Batch&, int, const Geo&, hipStream_t, const double2*, void*, double*, const void*,
                          const double2*, int) = nullptr;

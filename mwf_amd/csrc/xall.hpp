@@ -101,6 +101,11 @@ __global__ __launch_bounds__(xa_threads<LOGXA>()) void k_xall(Batch bt, const cp
                 lv[l][0] = pan[l * lstep];
                 lv[l][1] = pan[l * lstep + xstep];
             }
+        if (nlin == 4 && g.NLL > dev_lines(g.K0)) { // the vw share of E has a line of its own
+            const CT* pe = pan + (ptrdiff_t)(dev_lines(g.K0) + k - 1 - dev_line(k)) * lstep;
+            lv[DEV_E][0] = cadd(lv[DEV_E][0], pe[0]);
+            lv[DEV_E][1] = cadd(lv[DEV_E][1], pe[xstep]);
+        }
         if (item) {
 #pragma unroll
             for (int h = 0; h < 2; h++) {

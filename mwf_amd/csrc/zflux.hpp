@@ -54,19 +54,39 @@
 // would see.  With the profile in U the rounding of its unit-size constant
 // spread over every mode: the FP32 nonlinear term is 1.5 to 6 times closer to
 // the FP64 one this way (rms velocity 0.3 to 0.05).
-template <int K0_> struct Dev {
-    static constexpr int K0 = K0_, KK = 3 * K0 - 1;
-    static constexpr int NR = 5 * K0 - 3;     // real rows
-    static constexpr int NL = dev_lines(K0);  // output lines
+//
+// PART 0 is the whole pass.  PART 1, 2, 3 take the rows that need two of the
+// three components only (u w: uw and ww_0 - uu_0; u v: uv, vv - uu; v w: vw,
+// vv - ww), for rows so long that one block's registers do not hold all the base
+// values of its points; the vw share of E_k then goes to a line of its own, dev_lines +
+// k - 1, which the x kernel adds.
+template <int K0_, int PART = 0> struct Dev {
+    static constexpr int K0 = K0_;
+    // base lines, and the spec slot of base line i
+    static constexpr int NB = PART == 0 ? 3 * K0 - 1 : PART == 1 ? 2 * K0 : 2 * K0 - 1;
+    __host__ __device__ static constexpr int base(int i)
+    {
+        return PART == 1 ? (i < K0 ? i : i + K0 - 1) : PART == 3 ? i + K0 : i;
+    }
+    static constexpr int NR = PART == 0 ? 5 * K0 - 3 : PART == 1 ? K0 + 1 : 2 * K0 - 2; // real rows
+    static constexpr int NL = PART == 0 ? dev_lines(K0) : dev_lines_split(K0);          // lines of NL
     enum { UV, UW, VVUU, VW, VVWW, WWUU };
     __host__ __device__ static constexpr int k(int r) { return r < 2 ? 0 : 1 + (r - 2) / 5; }
     __host__ __device__ static constexpr int type(int r) { return r < 2 ? (r == 0 ? UW : WWUU) : (r - 2) % 5; }
-    __host__ __device__ static constexpr int order(int q) { return q < NR ? q : -1; }
+    // row at forward position q (two per complex sequence), -1 = padding
+    __host__ __device__ static constexpr int order(int q)
+    {
+        if (q >= NR) return -1;
+        if (PART == 0) return q;
+        if (PART == 1) return q < 2 ? q : 2 + 5 * (q - 2) + UW;
+        return 2 + 5 * (q / 2) + (PART == 2 ? (q & 1 ? VVUU : UV) : (q & 1 ? VVWW : VW));
+    }
     // uses of row r: line, kind (0: row, 1: ak row, 2: g row, 3: -i g row, 4: ak g row, 5: i (ak^2 - g^2) row)
     __host__ __device__ static constexpr int nuse(int r) { return type(r) == VW ? 2 : 1; }
     __host__ __device__ static constexpr int use_line(int r, int u)
     {
         const int t = type(r);
+        if (PART != 0 && t == VW && u == 0) return dev_lines(K0) + k(r) - 1;
         return dev_line(k(r)) + (t == UW ? DEV_UW : t == UV ? DEV_UV : t == VVUU || (t == VW && u == 0) ? DEV_E : DEV_F);
     }
     __host__ __device__ static constexpr int use_kind(int r, int u)
@@ -79,18 +99,18 @@ template <int K0_> struct Dev {
     // forward positions of the first and the last row of line L
     __host__ __device__ static constexpr int first(int L)
     {
-        for (int r = 0; r < NR; r++)
-            for (int u = 0; u < nuse(r); u++)
-                if (use_line(r, u) == L) return r;
+        for (int q = 0; q < NR; q++)
+            for (int u = 0; u < nuse(order(q)); u++)
+                if (use_line(order(q), u) == L) return q;
         return -1;
     }
     __host__ __device__ static constexpr int last(int L)
     {
-        int q = -1;
-        for (int r = 0; r < NR; r++)
-            for (int u = 0; u < nuse(r); u++)
-                if (use_line(r, u) == L) q = r;
-        return q;
+        int at = -1;
+        for (int q = 0; q < NR; q++)
+            for (int u = 0; u < nuse(order(q)); u++)
+                if (use_line(order(q), u) == L) at = q;
+        return at;
     }
 };
 
@@ -147,24 +167,21 @@ template <typename R, int LOGNN, int ZP, bool PP> constexpr size_t zc_lds_bytes(
                                 ptw_size<NN, 1, zc_pw<R, LOGNN, PP>()>() + (size_t)NN);
 }
 
-template <typename R, int K0, int LOGNN, int ZP, int WAVES, bool PP>
-__global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, const cplx_t<R>* __restrict__ U,
-                                                                   cplx_t<R>* __restrict__ NL,
-                                                                   const cplx_t<R>* __restrict__ twNN,
-                                                                   const cplx_t<R>* __restrict__ twQ)
+// the pass of block row xt (XB x-rows) over the rows of Dev<K0, PART>
+template <typename R, int K0, int PART, int LOGNN, int ZP, bool PP>
+__device__ __forceinline__ void zc_pass(const Geo& g, int xt, const cplx_t<R>* __restrict__ U, cplx_t<R>* __restrict__ NL,
+                                        const cplx_t<R>* __restrict__ twNN, const cplx_t<R>* __restrict__ twQ)
 {
     using CT = cplx_t<R>;
-    using FX = Dev<K0>;
+    using FX = Dev<K0, PART>;
     using FR = FluxRows<K0>;
-    const Geo g = bt.geo[blockIdx.z];
-    U += blockIdx.z * bt.u_stride;
-    NL += blockIdx.z * bt.nl_stride;
     constexpr int KK = 3 * K0 - 1;
+    constexpr int NB = FX::NB;
     constexpr int NN = 1 << LOGNN;
     constexpr int T = zc_threads<LOGNN>();
     constexpr int XB = T / NN;
     constexpr int H = NN / 2;
-    constexpr int NPI = (KK + 1) / 2;                 // inverse pairs: base lines 2p, 2p + 1
+    constexpr int NPI = (NB + 1) / 2;                 // inverse pairs: base lines 2p, 2p + 1
     constexpr int NBI = (NPI + ZP - 1) / ZP;
     constexpr int NR = FX::NR;
     constexpr int NPO = (NR + 1) / 2;                 // forward pairs: rows order(2p), order(2p + 1)
@@ -209,7 +226,7 @@ __global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, con
 
     const int tid = threadIdx.x;
     const int xl = tid >> LOGNN, r = tid & (NN - 1);
-    const int x0 = xcd_tile(blockIdx.x, gridDim.x) * XB;
+    const int x0 = xt * XB;
     const int x = x0 + xl;
     const bool valid = x < g.P;
     const bool wide = g.NTs * (int)sizeof(CT) >= 64;
@@ -232,12 +249,13 @@ __global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, con
             pf[f][0] = pf[f][1] = pf[f][2] = pf[f][3] = z;
             if (xg < g.P && pr < NPI) {
                 // U[x][line][n] with KK lines of NN (uidx, with the flux form's sizes)
-                const CT* u0 = U + ((size_t)(xg * KK + 2 * pr) << LOGNN);
+                const CT* u0 = U + ((size_t)(xg * KK + FX::base(2 * pr)) << LOGNN);
                 pf[f][0] = u0[fr];
                 pf[f][1] = u0[r2];
-                if (2 * pr + 1 < KK) {
-                    pf[f][2] = u0[NN + fr];
-                    pf[f][3] = u0[NN + r2];
+                if (2 * pr + 1 < NB) {
+                    const CT* u1 = PART == 1 ? U + ((size_t)(xg * KK + FX::base(2 * pr + 1)) << LOGNN) : u0 + NN;
+                    pf[f][2] = u1[fr];
+                    pf[f][3] = u1[r2];
                 }
             }
         }
@@ -291,8 +309,8 @@ __global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, con
 #pragma unroll
             for (int b = 0; b < 3; b++) {
                 const CT zv = buf[((xl * ZP + p) * 3 + b) * LPZ + lslot<LS>(r)];
-                vb[b][s1] = zv.x;
-                if constexpr (s1 + 1 < KK) vb[b][s1 + 1] = zv.y;
+                vb[b][FX::base(s1)] = zv.x;
+                if constexpr (s1 + 1 < NB) vb[b][FX::base(s1 + 1)] = zv.y;
             }
         });
         // with one buffer the next batch overwrites this one's results
@@ -363,7 +381,7 @@ __global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, con
 #pragma unroll
             for (int b = 0; b < 3; b++)
 #pragma unroll
-                for (int sl = 0; sl < KK; sl++) asm volatile("" : "+v"(vb[b][sl]));
+                for (int sl = 0; sl < NB; sl++) asm volatile("" : "+v"(vb[b][FX::base(sl)]));
             static_for<J0, J1>([&](auto ji) {
                 constexpr int j = decltype(ji)::value, q = j / 3, b = j % 3;
                 constexpr int r1 = FX::order(2 * q), r2 = FX::order(2 * q + 1);
@@ -425,7 +443,7 @@ __global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, con
 #pragma unroll
         for (int b = 0; b < 3; b++)
 #pragma unroll
-            for (int sl = 0; sl < KK; sl++) asm volatile("" : "+v"(vb[b][sl]));
+            for (int sl = 0; sl < NB; sl++) asm volatile("" : "+v"(vb[b][FX::base(sl)]));
         static_for<0, NV>([&](auto pi) {
             constexpr int p = decltype(pi)::value;
             constexpr int q1 = 2 * (RD * ZP + p);
@@ -464,4 +482,39 @@ __global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, con
         });
         if constexpr (!PP) __syncthreads();
     });
+}
+
+template <typename R, int K0, int LOGNN, int ZP, int WAVES, bool PP>
+__global__ __launch_bounds__(zc_threads<LOGNN>(), WAVES) void k_zc(Batch bt, const cplx_t<R>* __restrict__ U,
+                                                                   cplx_t<R>* __restrict__ NL,
+                                                                   const cplx_t<R>* __restrict__ twNN,
+                                                                   const cplx_t<R>* __restrict__ twQ)
+{
+    const Geo g = bt.geo[blockIdx.z];
+    zc_pass<R, K0, 0, LOGNN, ZP, PP>(g, xcd_tile(blockIdx.x, gridDim.x), U + blockIdx.z * bt.u_stride,
+                                     NL + blockIdx.z * bt.nl_stride, twNN, twQ);
+}
+
+// Rows of 1024 points in FP64: the points of a row hold more base values (M6:
+// 418 KB) than the registers of a block can keep beside its transforms, so three
+// blocks take the row, one for each pair of velocity components (Dev, PART 1 to
+// 3: 12, 11 and 11 base lines of M6).  They run back to back on one XCD (block B
+// on XCD B % 8; there part (B / 8) % 3 of row B / 24, each XCD a contiguous run
+// of rows) and read the row's U lines through its L2 once.  The 34 inverse line
+// transforms instead of 17 cost less than what the phase-sequential advective
+// kernel pays for reading and adding three partial sums of NL in memory.
+template <typename R, int K0, int LOGNN, int ZP>
+__global__ __launch_bounds__(zc_threads<LOGNN>(), 4) void k_zc3(Batch bt, const cplx_t<R>* __restrict__ U,
+                                                                cplx_t<R>* __restrict__ NL,
+                                                                const cplx_t<R>* __restrict__ twNN,
+                                                                const cplx_t<R>* __restrict__ twQ)
+{
+    const Geo g = bt.geo[blockIdx.z];
+    U += blockIdx.z * bt.u_stride;
+    NL += blockIdx.z * bt.nl_stride;
+    const int idx = blockIdx.x >> 3, nb = gridDim.x / 3, part = idx % 3;
+    const int xt = (blockIdx.x & 7) * (nb >> 3) + idx / 3;
+    if (part == 0) zc_pass<R, K0, 1, LOGNN, ZP, false>(g, xt, U, NL, twNN, twQ);
+    else if (part == 1) zc_pass<R, K0, 2, LOGNN, ZP, false>(g, xt, U, NL, twNN, twQ);
+    else zc_pass<R, K0, 3, LOGNN, ZP, false>(g, xt, U, NL, twNN, twQ);
 }
