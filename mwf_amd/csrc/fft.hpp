@@ -328,12 +328,19 @@ template <int L> constexpr int group_lanes() { return L / 8 < 64 ? L / 8 : 64; }
 // xo: a constant XORed into every slot of the group's region (a
 // per-sequence swizzle of the caller's layout; any xo < 16 keeps the access
 // patterns of the passes free of bank conflicts).  LS: the region's layout
-// (lslot; 0 = XOR swizzle, xo must be 0 otherwise).
-template <typename CT, int LOG, int SIGN, bool PTW = false, int PW = 3, int Ns = 1, int PASS = 0, int LS = 0>
+// (lslot; 0 = XOR swizzle, xo must be 0 otherwise).  BLK: a group of L/8 lanes
+// over several waves, 8 points per lane whatever L: block barriers take the
+// place of the wave's, every thread of the block makes the call, and the
+// caller puts a barrier between loading v from the region and the call.
+template <typename CT, int LOG, int SIGN, bool PTW = false, int PW = 3, int Ns = 1, int PASS = 0, int LS = 0, bool BLK = false>
 __device__ __forceinline__ void group_fft(CT* v, CT* __restrict__ reg, int gl, const CT* __restrict__ tw, int xo = 0)
 {
     constexpr int L = 1 << LOG;
-    constexpr int G = group_lanes<L>();
+    constexpr int G = BLK ? L / 8 : group_lanes<L>();
+    auto sync = [] {
+        if constexpr (BLK) __syncthreads();
+        else wave_lds_sync();
+    };
     if constexpr (Ns < L) {
         constexpr int R = radix_at<L, Ns>();
         constexpr int NBL = L / (R * G); // butterflies per lane
@@ -350,7 +357,7 @@ __device__ __forceinline__ void group_fft(CT* v, CT* __restrict__ reg, int gl, c
                 static_for<0, R>([&](auto ri) { x[i][ri] = lsw<decltype(ri)::value * (L / R), LS>(reg, pj); });
             }
         }
-        if constexpr (PASS > 0) wave_lds_sync();
+        if constexpr (PASS > 0 && !(BLK && LAST)) sync();
 #pragma unroll
         for (int i = 0; i < NBL; i++) {
             const int j = gl + G * i;
@@ -371,8 +378,8 @@ __device__ __forceinline__ void group_fft(CT* v, CT* __restrict__ reg, int gl, c
                 const int po = lslot<LS>((j - k) * R + k) ^ xo;
                 static_for<0, R>([&](auto ri) { lsw<decltype(ri)::value * Ns, LS>(reg, po) = x[i][ri]; });
             }
-            wave_lds_sync();
-            group_fft<CT, LOG, SIGN, PTW, PW, Ns * R, PASS + 1, LS>(v, reg, gl, tw, xo);
+            sync();
+            group_fft<CT, LOG, SIGN, PTW, PW, Ns * R, PASS + 1, LS, BLK>(v, reg, gl, tw, xo);
         }
     }
 }

@@ -1389,18 +1389,19 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
 // Fused x kernel of one step: forward x transform of NL, spec2mpt, AB2 and
 // implicit update of c and onl, then the inverse x transform of the updated
 // state for the next step's z kernel (mpt2spec + laminar + d/dx), so c is read
-// once per step.  Block (n-tile, y-mode k), XS = 3 * NT * G threads: each
-// group of G = min(64, MM/8) lanes owns one of the 3*NT sequences (t, b), 8
-// points per lane (16 at MM = 1024), and transforms it with group_fft (no
-// block barrier inside a transform); items (t, r), up to XTILE/XS per thread,
-// hold psi_k / phi_k at m = r and m = r - MM.  768 threads at every MM (at
-// MM = 1024, twice the 384 lanes of its six sequences).
+// once per step.  Block (n-tile, y-mode k), 768 threads: each group of MM/8
+// lanes owns one of the 3*NT sequences (t, b), 8 points per lane, and
+// transforms it with group_fft (for MM <= 512 with no block barrier inside a
+// transform); items (t, r), up to three per thread, hold psi_k / phi_k at m = r
+// and m = r - MM.
 // ---------------------------------------------------------------------------
-// Threads per block: one lane group per sequence, 3 XTILE/MM sequences; at MM
-// = 1024 (6 sequences) twice that, so that a thread holds 3 items instead of
-// 6 (the extra waves take items but no sequence).
-template <int LOGMM> constexpr int xs_mult() { return LOGMM >= 10 ? 2 : 1; }
-template <int LOGMM> constexpr int xs_of() { return xs_mult<LOGMM>() * 3 * (XTILE >> LOGMM) * group_lanes<(1 << LOGMM)>(); }
+// One group of MM/8 lanes per sequence, 8 points per lane.  At MM = 1024 a group
+// is two waves, whose transforms exchange with block barriers (group_fft, BLK):
+// with 16 points per lane on one wave, half the threads had no sequence and
+// the points left no registers for the new state, so that c was read again
+// (M6 2048^2 k_xstep 1436 -> 1171 us in FP64, 820 -> 739 in FP32; FP64 M4 MM =
+// 1024, NN = 256 232 -> 178).
+template <int LOGMM> constexpr int xs_of() { return 3 * XTILE / 8; }
 
 // FP32 k_xstep streams the next NL panel straight into an LDS staging area
 // (global_load_lds, no registers) while the current line is transformed: the
@@ -1447,29 +1448,28 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
 {
     using CT = cplx_t<R>;
     constexpr int MM = 1 << LOGMM;
-    constexpr int G = group_lanes<MM>();
-    constexpr int PL = MM / G;
+    constexpr int G = MM / 8;
+    constexpr int PL = 8;
     constexpr int XS = xs_of<LOGMM>();
     constexpr int IPT = (XTILE + XS - 1) / XS; // items per thread
     constexpr int LPT = 3 * XTILE / XS;        // rows per thread in the cooperative load/store
     // After the update each thread holds the new state of its items in
-    // psi/phi; the inverse half rebuilds its 6 lines from those registers
+    // psi/phi; the inverse half rebuilds its lines from those registers
     // instead of re-reading c (k_xstep 10 % faster in FP64, 18 % in FP32 at
-    // MM = 512).  At MM = 1024 (6 items per thread) the registers spill and
-    // the kernel re-reads c instead.
-    constexpr bool XREG = !INV_ONLY && LOGMM < 10;
+    // MM = 512).
+    constexpr bool XREG = !INV_ONLY;
+    constexpr bool BLK = LOGMM >= 10; // transforms of more than one wave
     extern __shared__ unsigned char smem_raw[];
     CT* reg = reinterpret_cast<CT*>(smem_raw); // [XS/G sequences][MM], swizzled
     CT* twMl = reg + 3 * XTILE;                // pass twiddles of the MM-point transforms (seven-entry)
     static_assert(ptw_size<MM, 1, 7>() % 2 == 0, "twPl must stay 16-byte aligned");
     double2* twPl = reinterpret_cast<double2*>(twMl + ptw_size<MM, 1, 7>()); // exp(2 pi i j/P), j <= 2 MM
     constexpr bool ASYNC = xstep_async<R>() && !INV_ONLY;
-    // FP32 at MM <= 512: the forward transforms' first pass reads a whole
+    // FP32: the forward transforms' first pass reads a whole
     // tile's sequences straight from the staged panel (element a of sequence
     // (t, b) at panel row 3a + b, column t), with no copy into the transform
-    // layout and no barrier between (k_xstep 0.130 -> 0.123 ms at M4 1024^2);
-    // at MM = 1024 that form spills 32 VGPRs and is 30 % slower
-    constexpr bool SREAD = ASYNC && LOGMM < 10;
+    // layout and no barrier between (k_xstep 0.130 -> 0.123 ms at M4 1024^2)
+    constexpr bool SREAD = ASYNC;
     CT* stage = reinterpret_cast<CT*>(twPl + 2 * MM + 1);               // [3 XTILE] next NL panel
 
     const Geo g = bt.geo[blockIdx.z];
@@ -1485,7 +1485,7 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
     const int nitems = NT * MM;
     const int nrows = 3 * nitems; // (x, t) pairs of one line
     const int s = tid / G, gl = tid % G;
-    const bool seq_on = s < 3 * NT;
+    const bool seq_on = BLK || s < 3 * NT; // NT is whole at MM = 1024 (NN >= 16)
     CT* myreg = reg + s * MM;
     const int sxo = xsw<R>(s / 3, s % 3); // swizzle of this thread's group sequence
     // Decimating transposes between a panel ([x][t], i = x NT + t, x = 3a + b)
@@ -1616,7 +1616,9 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
                 } else {
                     static_for<0, PL>([&](auto qi) { v[qi] = swz<decltype(qi)::value * G>(myreg, pg); });
                 }
-                group_fft<CT, LOGMM, -1, true, 7>(v, myreg, gl, twMl, sxo);
+                if constexpr (BLK && !SREAD) __syncthreads();
+                group_fft<CT, LOGMM, -1, true, 7, 1, 0, 0, BLK>(v, myreg, gl, twMl, sxo);
+                if constexpr (BLK) __syncthreads();
                 static_for<0, PL>([&](auto qi) { swz<decltype(qi)::value * G>(myreg, pg) = v[qi]; });
             }
             __syncthreads();
@@ -1764,7 +1766,9 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
             CT v[PL];
             const int pg = pidx(gl) ^ sxo;
             static_for<0, PL>([&](auto qi) { v[qi] = swz<decltype(qi)::value * G>(myreg, pg); });
-            group_fft<CT, LOGMM, +1, true, 7>(v, myreg, gl, twMl, sxo);
+            if constexpr (BLK) __syncthreads();
+            group_fft<CT, LOGMM, +1, true, 7, 1, 0, 0, BLK>(v, myreg, gl, twMl, sxo);
+            if constexpr (BLK) __syncthreads();
             static_for<0, PL>([&](auto qi) { swz<decltype(qi)::value * G>(myreg, pg) = v[qi]; });
         }
         __syncthreads();
