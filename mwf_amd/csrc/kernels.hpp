@@ -1128,7 +1128,7 @@ __device__ __forceinline__ void s2m_finish(int k, int mi, int n, double2 u, doub
 }
 
 // Flux form: the share of line type li (uw, F, uv, E of wall-normal index k,
-// zflux.hpp; not yet scaled by 1/(PQ)) in psi_k and phi_k of the nonlinear term
+// zflux.hpp; not yet scaled, dev_scale) in psi_k and phi_k of the nonlinear term
 // at one (m, n), from the line's forward x transform X; rak = 1/ak1, for k = 0
 // -1 (F_0 has the multiplier a).  At (0,0), where every multiplier vanishes, the
 // mean-mode rows of var_spec2mpt apply instead: psi = -N_u = -ak uv, phi = -N_w =
@@ -1162,6 +1162,10 @@ __device__ __forceinline__ void dev_term(int li, bool mean, double2 X, double am
         if (li == DEV_F) phi = double2{-(X.y * rak), X.x * rak};
     }
 }
+
+// scale of the flux form's lines: 1/(PQ), and 1/2 of the split of two real rows,
+// which the z kernels leave out (exact)
+__device__ __forceinline__ double dev_scale(const Geo& g) { return 0.5 * g.scale; }
 
 // Radix-3 unfold of the padded forward x transform, X[m] = sum_b w^{-mb} F_b[m
 // mod MM] at m = r (Xp) and m = r - MM (Xn), tw[j] = exp(2 pi i j/P).  Fused
@@ -1367,7 +1371,7 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
                 const int slot = which == 0 ? k : g.K0 - 1 + k;
                 const size_t idx = ((size_t)n * g.K + slot) * g.ldM + mi;
                 double2 nl = which == 0 ? psi[q][h] : phi[q][h];
-                if constexpr (FLUX) nl = double2{nl.x * g.scale, nl.y * g.scale};
+                if constexpr (FLUX) nl = double2{nl.x * dev_scale(g), nl.y * dev_scale(g)};
                 if (mode == 1) {
                     nlout[idx] = nl;
                     continue;
@@ -1686,7 +1690,7 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
                     const int slot = which == 0 ? k : g.K0 - 1 + k;
                     const size_t idx = ((size_t)n * g.K + slot) * g.ldM + mi;
                     double2 nl = which == 0 ? psi[q][h] : phi[q][h];
-                    if constexpr (FLUX) nl = double2{nl.x * g.scale, nl.y * g.scale};
+                    if constexpr (FLUX) nl = double2{nl.x * dev_scale(g), nl.y * dev_scale(g)};
                     double lhs, rhs;
                     lhsrhs_k(g, k, which, mean, am2, an2, ak2, lhs, rhs);
                     const double2 cv = c[idx];

@@ -163,7 +163,7 @@ __global__ __launch_bounds__(xa_threads<LOGXA>()) void k_xall(Batch bt, const cp
                     if (which == 1 && k == 0) continue;
                     const size_t idx = (which == 0 ? cpsi : cphi) + mi;
                     double2 nl = which == 0 ? psi[h] : phi[h];
-                    nl = double2{nl.x * g.scale, nl.y * g.scale};
+                    nl = double2{nl.x * dev_scale(g), nl.y * dev_scale(g)};
                     double lhs, rhs;
                     lhsrhs_k(g, k, which, mean, am2, an2, ak2, lhs, rhs);
                     const double2 old = nst ? nl : hist_wide(ov[h][which]);

@@ -165,11 +165,11 @@ __global__ __launch_bounds__((zs_threads<K0, LOGNN>())) void k_zs(Batch bt, cons
         if (k >= K0) continue;
         const int pn = lslot<LS>(n), pm = lslot<LS>(nm);
         const CT w1 = cconj(twQl[n]), w2 = cconj(twq2<R>(twQl, NN, 2 * n));
-        // transforms of the two real sequences of complex sequence s
+        // twice the transforms of the two real sequences of complex sequence s
         auto split = [&](const CT* s, CT& F1, CT& F2) {
             const CT zn = s[pn], zm = s[pm];
-            F1 = CT{(R)0.5 * (zn.x + zm.x), (R)0.5 * (zn.y - zm.y)};
-            F2 = CT{(R)0.5 * (zn.y + zm.y), (R)0.5 * (zm.x - zn.x)};
+            F1 = CT{zn.x + zm.x, zn.y - zm.y};
+            F2 = CT{zn.y + zm.y, zm.x - zn.x};
         };
         // rows X1, X2 of the pair whose phases are the sequences s, s + 1, s + 2
         auto pair = [&](const CT* s, CT& X1, CT& X2) {

@@ -18,7 +18,7 @@
 //
 // so five real rows per k >= 1 (uv, uw, vv - uu, vw, vv - ww; two for k = 0) are
 // transformed forward, and four lines per k >= 1 (uw, F, uv, E; two for k = 0)
-// cross to the x kernel, which applies the powers of a and the scale 1/(PQ)
+// cross to the x kernel, which applies the powers of a and the scale 1/(2 PQ)
 // (Dev below, and dev_term in kernels.hpp): M4 17 rows and 14 lines, M6 27 and
 // 22.  The form with one line to be differentiated in x and one for the rest per
 // spec slot has 21 rows and 22 lines (33 and 34), so 36 % of NL's bytes and of
@@ -280,6 +280,18 @@ __device__ __forceinline__ void zc_pass(const Geo& g, int xt, const cplx_t<R>* _
         return t;
     };
 
+    // A thread's fold tasks have one index fr, its output one r: where registers
+    // allow, the twiddles of the folds and then of the unfolds are looked up once
+    constexpr bool HT = PP && T % H == 0;
+    CT tf[4];
+    if constexpr (HT) {
+        const int fr = tid % H, fm = fr == 0 ? H : NN - fr;
+        tf[0] = twQl[fr];
+        tf[1] = twQl[fm];
+        tf[2] = twq2<R>(twQl, NN, 2 * fr);
+        tf[3] = twq2<R>(twQl, NN, 2 * fm);
+    }
+
     // ---- inverse z transforms of the base lines (c2r, +1) ----
     static_for<0, NBI>([&](auto bi) {
         constexpr int BN = decltype(bi)::value;
@@ -296,9 +308,14 @@ __device__ __forceinline__ void zc_pass(const Geo& g, int xt, const cplx_t<R>* _
             CT* seq = buf + ((fx * ZP + fp) * 3) * LPZ;
             const CT one{(R)1, (R)0};
             zfold_bw<R, LS>(seq, 0, fr, NN, pf[f][0], pf[f][1], pf[f][2], pf[f][3], one, one);
-            zfold_bw<R, LS>(seq + LPZ, 1, fr, NN, pf[f][0], pf[f][1], pf[f][2], pf[f][3], twQl[fr], twQl[fm]);
-            zfold_bw<R, LS>(seq + 2 * LPZ, 2, fr, NN, pf[f][0], pf[f][1], pf[f][2], pf[f][3], twq2<R>(twQl, NN, 2 * fr),
-                        twq2<R>(twQl, NN, 2 * fm));
+            if constexpr (HT) {
+                zfold_bw<R, LS>(seq + LPZ, 1, fr, NN, pf[f][0], pf[f][1], pf[f][2], pf[f][3], tf[0], tf[1]);
+                zfold_bw<R, LS>(seq + 2 * LPZ, 2, fr, NN, pf[f][0], pf[f][1], pf[f][2], pf[f][3], tf[2], tf[3]);
+            } else {
+                zfold_bw<R, LS>(seq + LPZ, 1, fr, NN, pf[f][0], pf[f][1], pf[f][2], pf[f][3], twQl[fr], twQl[fm]);
+                zfold_bw<R, LS>(seq + 2 * LPZ, 2, fr, NN, pf[f][0], pf[f][1], pf[f][2], pf[f][3],
+                                twq2<R>(twQl, NN, 2 * fr), twq2<R>(twQl, NN, 2 * fm));
+            }
         }
         if constexpr (BN + 1 < NBI) prefetch(BN + 1);
         __syncthreads();
@@ -322,6 +339,11 @@ __device__ __forceinline__ void zc_pass(const Geo& g, int xt, const cplx_t<R>* _
     const R beta = (R)g.beta, bg = (R)(g.beta * (g.gamma * r));
     const R b2 = (R)(g.beta * g.beta), g2 = (R)((g.gamma * r) * (g.gamma * r));
     const R lu = (R)g.cth, lw = (R)g.sth; // laminar u_1, w_1
+    if constexpr (HT) {
+        tf[0] = cconj(twQl[r]);
+        tf[1] = cconj(twq2<R>(twQl, NN, 2 * r));
+    }
+    auto unfold_tw = [&](int b, int rv) { return HT ? tf[b - 1] : cconj(twq2<R>(twQl, NN, rv * b)); };
     constexpr int NLN = FX::NL;          // lines of NL
     CT acc[NLN];
     // line assembly of the two rows q1, q1 + 1 of a forward pair from their
@@ -401,14 +423,14 @@ __device__ __forceinline__ void zc_pass(const Geo& g, int xt, const cplx_t<R>* _
                 constexpr int j = decltype(ji)::value, q = j / 3, b = j % 3;
                 const CT zn = buf[(j - J0) * LPZ + lslot<LS>(r)];
                 const CT zm = buf[(j - J0) * LPZ + lslot<LS>(rm)];
-                const CT F1 = CT{(R)0.5 * (zn.x + zm.x), (R)0.5 * (zn.y - zm.y)};
-                const CT F2 = CT{(R)0.5 * (zn.y + zm.y), (R)0.5 * (zm.x - zn.x)};
+                const CT F1 = CT{zn.x + zm.x, zn.y - zm.y};
+                const CT F2 = CT{zn.y + zm.y, zm.x - zn.x};
                 if constexpr (LONE && q == QL) {
                     if constexpr (b == 0) { // phase 0 (F1) and phase 1 (F2) of the one row
-                        X[0] = cadd(F1, cmul(F2, cconj(twq2<R>(twQl, NN, r))));
+                        X[0] = cadd(F1, cmul(F2, unfold_tw(1, r)));
                         X[1] = CT{(R)0, (R)0};
                     } else { // phase 2
-                        X[0] = cadd(X[0], cmul(F1, cconj(twq2<R>(twQl, NN, 2 * r))));
+                        X[0] = cadd(X[0], cmul(F1, unfold_tw(2, r)));
                         assemble(std::integral_constant<int, 2 * q>{}, X, nlr, nls);
                     }
                 } else {
@@ -416,7 +438,7 @@ __device__ __forceinline__ void zc_pass(const Geo& g, int xt, const cplx_t<R>* _
                         X[0] = F1;
                         X[1] = F2;
                     } else {
-                        const CT w = cconj(twq2<R>(twQl, NN, r * b));
+                        const CT w = unfold_tw(b, r);
                         X[0] = cadd(X[0], cmul(F1, w));
                         X[1] = cadd(X[1], cmul(F2, w));
                     }
@@ -467,13 +489,13 @@ __device__ __forceinline__ void zc_pass(const Geo& g, int xt, const cplx_t<R>* _
             for (int b = 0; b < 3; b++) {
                 const CT zn = buf[((xl * ZP + p) * 3 + b) * LPZ + lslot<LS>(r)];
                 const CT zm = buf[((xl * ZP + p) * 3 + b) * LPZ + lslot<LS>(rm)];
-                const CT F1 = CT{(R)0.5 * (zn.x + zm.x), (R)0.5 * (zn.y - zm.y)};
-                const CT F2 = CT{(R)0.5 * (zn.y + zm.y), (R)0.5 * (zm.x - zn.x)};
+                const CT F1 = CT{zn.x + zm.x, zn.y - zm.y};
+                const CT F2 = CT{zn.y + zm.y, zm.x - zn.x};
                 if (b == 0) {
                     X[0] = F1;
                     X[1] = F2;
                 } else {
-                    const CT w = cconj(twq2<R>(twQl, NN, r * b));
+                    const CT w = unfold_tw(b, r);
                     X[0] = cadd(X[0], cmul(F1, w));
                     X[1] = cadd(X[1], cmul(F2, w));
                 }
