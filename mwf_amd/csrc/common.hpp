@@ -122,13 +122,16 @@ __device__ __forceinline__ size_t uidx(const Geo& g, int x, int line, int n)
 {
     return ((size_t)x * g.UL + line) * g.NN + n;
 }
-// NL stripe of an x-kernel block (columns n0 .. n0 + NTx - 1, slot): element
-// i = x * NTx + t at offset pan_at(g, i) from the returned base.
+// NL stripe of an x-kernel block (columns n0 .. n0 + NT - 1, slot): element
+// i = x * NT + t at offset pan_at(g, log2(NT), i) from the returned base.
 template <typename CT> __device__ __forceinline__ const CT* nl_panel(const Geo& g, const CT* NL, int n0, int slot)
 {
     return NL + ((size_t)(n0 >> g.lgNS) * g.NLL + slot) * g.P * g.NTs + (n0 & (g.NTs - 1));
 }
-__device__ __forceinline__ int pan_at(const Geo& g, int i) { return ((i >> g.lgNT) << g.lgNS) + (i & (g.NTx - 1)); }
+__device__ __forceinline__ int pan_at(const Geo& g, int lgNT, int i)
+{
+    return ((i >> lgNT) << g.lgNS) + (i & ((1 << lgNT) - 1));
+}
 __device__ __forceinline__ size_t nidx(const Geo& g, int x, int slot, int n)
 {
     const int tile = n >> g.lgNS, t = n & (g.NTs - 1);

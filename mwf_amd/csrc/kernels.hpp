@@ -1299,7 +1299,7 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
             if (it >= 3 * nitems) continue;
             const int x = it >> g.lgNT, t = it & (NT - 1);
             const int a = x / 3, b = x - 3 * a;
-            const int po = pan_at(g, it);
+            const int po = pan_at(g, g.lgNT, it);
             CT v = pan[po];
             if (FLUX && li == DEV_E && g.NLL > dev_lines(g.K0)) // the vw share of E
                 v = cadd(v, pan[po + evw]);
@@ -1405,7 +1405,7 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
 // the points left no registers for the new state, so that c was read again
 // (M6 2048^2 k_xstep 1436 -> 1171 us in FP64, 820 -> 739 in FP32; FP64 M4 MM =
 // 1024, NN = 256 232 -> 178).
-template <int LOGMM> constexpr int xs_of() { return 3 * XTILE / 8; }
+template <int LXT = LOG_XTILE> constexpr int xs_of() { return (3 << LXT) / 8; }
 
 // FP32 k_xstep streams the next NL panel straight into an LDS staging area
 // (global_load_lds, no registers) while the current line is transformed: the
@@ -1424,7 +1424,10 @@ template <typename R> __device__ __forceinline__ int xsw(int t, int b)
     if constexpr (sizeof(R) == 4) return ((t * 9) ^ (b * 3)) & 15; // 8-byte slots, 16 per bank phase
     else return ((t * 5) ^ b) & 7;                                 // 16-byte slots, 8 per bank phase
 }
-template <typename R> constexpr size_t xstep_stage_bytes() { return xstep_async<R>() ? 3 * (size_t)XTILE * sizeof(cplx_t<R>) : 0; }
+template <typename R, int LXT = LOG_XTILE> constexpr size_t xstep_stage_bytes()
+{
+    return xstep_async<R>() ? ((size_t)3 << LXT) * sizeof(cplx_t<R>) : 0;
+}
 
 // Wave-cooperative copy of a block's NL stripe (nch 16-byte chunks, chunk c
 // holding stripe elements c E .. c E + E - 1, E = 16 / sizeof(CT), which lie
@@ -1433,19 +1436,21 @@ template <typename R> constexpr size_t xstep_stage_bytes() { return xstep_async<
 // the wave.  nch is a multiple of 64.  The data is in LDS once the wave's
 // vector memory count has drained and a barrier has passed.
 template <int T, typename CT>
-__device__ __forceinline__ void panel_to_lds(const Geo& g, const CT* __restrict__ src, CT* dst, int nch, int tid)
+__device__ __forceinline__ void panel_to_lds(const Geo& g, int lgNT, const CT* __restrict__ src, CT* dst, int nch, int tid)
 {
     constexpr int E = 16 / (int)sizeof(CT);
     const int wave = tid >> 6, lane = tid & 63;
     char* l = reinterpret_cast<char*>(dst);
     for (int c0 = wave * 64; c0 < nch; c0 += T)
-        __builtin_amdgcn_global_load_lds(reinterpret_cast<const char*>(src + pan_at(g, (c0 + lane) * E)),
+        __builtin_amdgcn_global_load_lds(reinterpret_cast<const char*>(src + pan_at(g, lgNT, (c0 + lane) * E)),
                                          (__attribute__((address_space(3))) void*)(l + (size_t)c0 * 16), 16, 0, 0);
 }
 __device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-template <typename R, int LOGMM, bool INV_ONLY, bool FLUX>
-__global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t<R>* __restrict__ NL, double2* __restrict__ c,
+// LXT: log2 of the values of a line in the tile (XTILE; smaller tiles only where NN
+// fills them and MM <= 512)
+template <typename R, int LOGMM, bool INV_ONLY, bool FLUX, int LXT = LOG_XTILE>
+__global__ __launch_bounds__(xs_of<LXT>(), 3) void k_xstep(Batch bt, const cplx_t<R>* __restrict__ NL, double2* __restrict__ c,
                                               cplx_t<R>* __restrict__ onl, cplx_t<R>* __restrict__ U,
                                               const cplx_t<R>* __restrict__ twMM, const double2* __restrict__ twP,
                                               int nst)
@@ -1454,9 +1459,10 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
     constexpr int MM = 1 << LOGMM;
     constexpr int G = MM / 8;
     constexpr int PL = 8;
-    constexpr int XS = xs_of<LOGMM>();
-    constexpr int IPT = (XTILE + XS - 1) / XS; // items per thread
-    constexpr int LPT = 3 * XTILE / XS;        // rows per thread in the cooperative load/store
+    constexpr int XTL = 1 << LXT;             // values of a line in the tile
+    constexpr int XS = xs_of<LXT>();
+    constexpr int IPT = (XTL + XS - 1) / XS; // items per thread
+    constexpr int LPT = 3 * XTL / XS;        // rows per thread in the cooperative load/store
     // After the update each thread holds the new state of its items in
     // psi/phi; the inverse half rebuilds its lines from those registers
     // instead of re-reading c (k_xstep 10 % faster in FP64, 18 % in FP32 at
@@ -1465,7 +1471,7 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
     constexpr bool BLK = LOGMM >= 10; // transforms of more than one wave
     extern __shared__ unsigned char smem_raw[];
     CT* reg = reinterpret_cast<CT*>(smem_raw); // [XS/G sequences][MM], swizzled
-    CT* twMl = reg + 3 * XTILE;                // pass twiddles of the MM-point transforms (seven-entry)
+    CT* twMl = reg + 3 * XTL;                // pass twiddles of the MM-point transforms (seven-entry)
     static_assert(ptw_size<MM, 1, 7>() % 2 == 0, "twPl must stay 16-byte aligned");
     double2* twPl = reinterpret_cast<double2*>(twMl + ptw_size<MM, 1, 7>()); // exp(2 pi i j/P), j <= 2 MM
     constexpr bool ASYNC = xstep_async<R>() && !INV_ONLY;
@@ -1474,7 +1480,7 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
     // (t, b) at panel row 3a + b, column t), with no copy into the transform
     // layout and no barrier between (k_xstep 0.130 -> 0.123 ms at M4 1024^2)
     constexpr bool SREAD = ASYNC;
-    CT* stage = reinterpret_cast<CT*>(twPl + 2 * MM + 1);               // [3 XTILE] next NL panel
+    CT* stage = reinterpret_cast<CT*>(twPl + 2 * MM + 1);               // [3 XTL] next NL panel
 
     const Geo g = bt.geo[blockIdx.z];
     NL += blockIdx.z * bt.nl_stride;
@@ -1482,7 +1488,7 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
     onl += blockIdx.z * bt.c_stride;
     U += blockIdx.z * bt.u_stride;
 
-    const int NT = g.NTx;
+    const int lgNT = LXT == LOG_XTILE ? g.lgNT : LXT - LOGMM, NT = 1 << lgNT;
     const int n0 = xcd_tile(blockIdx.x, gridDim.x) * NT;
     const int k = blockIdx.y;
     const int tid = threadIdx.x;
@@ -1498,7 +1504,7 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
     // a = a0 + DA q (DA = XS / (3 NTC), a power of two above a0), so its slot
     // is one per-thread base and a constant (swz); otherwise every item's
     // indices are computed.
-    constexpr int NTC = XTILE >> LOGMM, LOGNTC = LOG_XTILE - LOGMM;
+    constexpr int NTC = XTL >> LOGMM, LOGNTC = LXT - LOGMM;
     constexpr int DA = XS / (3 * NTC);
     static_assert((1 << LOGNTC) == NTC && XS == 3 * NTC * DA && (DA & (DA - 1)) == 0, "whole-tile transposes");
     const bool whole = NT == NTC;
@@ -1534,7 +1540,7 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
             return nl_panel(g, NL, n0, slot);
         };
         const int nch = nrows * (int)sizeof(CT) / 16; // 16-byte chunks of one stripe
-        if constexpr (ASYNC) panel_to_lds<XS>(g, panel_of(0), stage, nch, tid);
+        if constexpr (ASYNC) panel_to_lds<XS>(g, lgNT, panel_of(0), stage, nch, tid);
 #pragma unroll 1
         for (int li = 0; li < NLI; li++) {
             if (!line_on(li)) continue;
@@ -1561,7 +1567,7 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
                         for (int q = 0; q < LPT; q++) {
                             const int i = tidv + XS * q;
                             if (i >= nrows) continue;
-                            const int x = i >> g.lgNT, t = i & (NT - 1);
+                            const int x = i >> lgNT, t = i & (NT - 1);
                             const int a = x / 3, b = x - 3 * a;
                             reg[(t * 3 + b) * MM + (pidx(a) ^ xsw<R>(t, b))] = stage[i];
                         }
@@ -1569,7 +1575,7 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
                     __syncthreads();
                     int ln = li + 1;
                     while (ln < NLI && !line_on(ln)) ln++;
-                    if (ln < NLI) panel_to_lds<XS>(g, panel_of(ln), stage, nch, tid);
+                    if (ln < NLI) panel_to_lds<XS>(g, lgNT, panel_of(ln), stage, nch, tid);
                 }
             } else {
                 const CT* pan = panel_of(li);
@@ -1591,7 +1597,7 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
                     tile_item(tidv, t0, xq, rb, pa);
                     // item q is element tidv + XS q of the stripe: XS/NTx
                     // x-rows further
-                    const CT* pb = pan + pan_at(g, tidv);
+                    const CT* pb = pan + pan_at(g, lgNT, tidv);
                     const int pstep = (XS >> LOGNTC) << g.lgNS;
                     static_for<0, LPT>([&](auto qi) {
                         constexpr int q = decltype(qi)::value;
@@ -1602,9 +1608,9 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
                     for (int q = 0; q < LPT; q++) {
                         const int i = tidv + XS * q;
                         if (i >= nrows) continue;
-                        const int x = i >> g.lgNT, t = i & (NT - 1);
+                        const int x = i >> lgNT, t = i & (NT - 1);
                         const int a = x / 3, b = x - 3 * a;
-                        reg[(t * 3 + b) * MM + (pidx(a) ^ xsw<R>(t, b))] = nl_at(pan + pan_at(g, i));
+                        reg[(t * 3 + b) * MM + (pidx(a) ^ xsw<R>(t, b))] = nl_at(pan + pan_at(g, lgNT, i));
                     }
                 }
                 __syncthreads();
@@ -1630,7 +1636,7 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
                 if (whole) { // the staged panel has been read: start the next line's
                     int ln = li + 1;
                     while (ln < NLI && !line_on(ln)) ln++;
-                    if (ln < NLI) panel_to_lds<XS>(g, panel_of(ln), stage, nch, tid);
+                    if (ln < NLI) panel_to_lds<XS>(g, lgNT, panel_of(ln), stage, nch, tid);
                 }
             }
 #pragma unroll
@@ -1709,7 +1715,7 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
         }
     }
 
-    const bool wide = g.NTx * (int)sizeof(CT) >= 64;
+    const bool wide = NT * (int)sizeof(CT) >= 64;
     // ---------------- inverse x transform of the new state ----------------
 #pragma unroll 1
     for (int li = 0; li < (FLUX ? 3 : 6); li++) {
@@ -1793,7 +1799,7 @@ __global__ __launch_bounds__(xs_of<LOGMM>()) void k_xstep(Batch bt, const cplx_t
             for (int q = 0; q < LPT; q++) {
                 const int i = tidv + XS * q;
                 if (i >= nrows) continue;
-                const int x = i >> g.lgNT, t = i & (NT - 1);
+                const int x = i >> lgNT, t = i & (NT - 1);
                 const int a = x / 3, b = x - 3 * a;
                 st_piece(Ul + x * ustride + t, reg[(t * 3 + b) * MM + (pidx(a) ^ xsw<R>(t, b))], wide);
             }

@@ -35,24 +35,25 @@ static hipError_t launch_xfwd(const Batch& bt, int nmem, const Geo& g, hipStream
 
 // transform buffers, then the pass twiddles of the MM-point transforms and
 // 2 MM + 1 fold twiddles
-template <typename R, int LOGMM> static size_t xstep_lds()
+template <typename R, int LOGMM, int LXT = LOG_XTILE> static size_t xstep_lds()
 {
     constexpr size_t MM = (size_t)1 << LOGMM;
-    return (3 * (size_t)XTILE + ptw_size<(1 << LOGMM), 1, 7>()) * sizeof(cplx_t<R>) +
-           (2 * MM + 1) * sizeof(double2) + xstep_stage_bytes<R>();
+    return (((size_t)3 << LXT) + ptw_size<(1 << LOGMM), 1, 7>()) * sizeof(cplx_t<R>) + (2 * MM + 1) * sizeof(double2) +
+           xstep_stage_bytes<R, LXT>();
 }
 
-template <typename R, int LOGMM, bool FLUX>
+template <typename R, int LOGMM, bool FLUX, int LXT = LOG_XTILE>
 static hipError_t launch_xstep(const Batch& bt, int nmem, const Geo& g, hipStream_t s, const void* NL, double2* c,
                                void* onl, void* U, const void* twMM, const double2* twP, int nst, int inv_only)
 {
     using CT = cplx_t<R>;
-    dim3 grid(g.NN / g.NTx, g.K0, nmem);
+    dim3 grid(LXT == LOG_XTILE ? g.NN / g.NTx : g.NN >> (LXT - LOGMM), g.K0, nmem);
+    const size_t lds = xstep_lds<R, LOGMM, LXT>();
     if (inv_only)
-        hipLaunchKernelGGL((k_xstep<R, LOGMM, true, FLUX>), grid, dim3(xs_of<LOGMM>()), (xstep_lds<R, LOGMM>()), s, bt, (const CT*)NL,
+        hipLaunchKernelGGL((k_xstep<R, LOGMM, true, FLUX, LXT>), grid, dim3(xs_of<LXT>()), lds, s, bt, (const CT*)NL,
                            c, (CT*)onl, (CT*)U, (const CT*)twMM, twP, nst);
     else
-        hipLaunchKernelGGL((k_xstep<R, LOGMM, false, FLUX>), grid, dim3(xs_of<LOGMM>()), (xstep_lds<R, LOGMM>()), s, bt, (const CT*)NL,
+        hipLaunchKernelGGL((k_xstep<R, LOGMM, false, FLUX, LXT>), grid, dim3(xs_of<LXT>()), lds, s, bt, (const CT*)NL,
                            c, (CT*)onl, (CT*)U, (const CT*)twMM, twP, nst);
     return hipGetLastError();
 }
@@ -74,17 +75,21 @@ static hipError_t launch_xall(const Batch& bt, int nmem, const Geo& g, hipStream
 }
 
 // the fused x kernel of the flux form: k_xall or k_xstep by the size of the launch
-template <typename R, int LOGMM, int LX = 9>
+template <typename R, int LOGMM, int LX = 10>
 static hipError_t launch_xf(const Batch& bt, int nmem, const Geo& g, hipStream_t s, const void* NL, double2* c,
                             void* onl, void* U, const void* twMM, const double2* twP, int nst, int inv_only)
 {
-    if constexpr (LX >= 6 && LX >= LOGMM && LOGMM <= 9) {
-        int lx = xall_log<LOGMM>((g.NN / g.NTx) * g.K0 * nmem);
-        while (lx > LOGMM && (1 << (lx - LOGMM)) > g.NN) lx--; // whole tiles
-        if (lx == LX) return launch_xall<R, LOGMM, LX>(bt, nmem, g, s, NL, c, onl, U, twMM, twP, nst, inv_only);
+    if constexpr (LX < 6 || LX < LOGMM || LOGMM > 9)
+        return launch_xstep<R, LOGMM, true>(bt, nmem, g, s, NL, c, onl, U, twMM, twP, nst, inv_only);
+    else {
+        if (xtile_log<R, LOGMM>((g.NN / g.NTx) * g.K0 * nmem, g.NN) == LX) {
+            if constexpr (LX <= 9)
+                return launch_xall<R, LOGMM, LX>(bt, nmem, g, s, NL, c, onl, U, twMM, twP, nst, inv_only);
+            else if constexpr (LOGMM >= 6)
+                return launch_xstep<R, LOGMM, true, LX>(bt, nmem, g, s, NL, c, onl, U, twMM, twP, nst, inv_only);
+        }
         return launch_xf<R, LOGMM, LX - 1>(bt, nmem, g, s, NL, c, onl, U, twMM, twP, nst, inv_only);
     }
-    return launch_xstep<R, LOGMM, true>(bt, nmem, g, s, NL, c, onl, U, twMM, twP, nst, inv_only);
 }
 
 template <typename R, int LOGMM>
@@ -164,6 +169,10 @@ template <typename R> void prepare_x(int lm)
         set_lds(k_xstep<R, L, false, true>, xstep_lds<R, L>());  \
         set_lds(k_xstep<R, L, true, true>, xstep_lds<R, L>());   \
         prep_xall<R, L>();                             \
+        if constexpr (L >= 6) {                        \
+            set_lds(k_xstep<R, L, false, true, 10>, xstep_lds<R, L, 10>()); \
+            set_lds(k_xstep<R, L, true, true, 10>, xstep_lds<R, L, 10>());  \
+        }                                              \
         set_lds(k_sxinv<R, L>, x_lds<R, L>());         \
         set_lds(k_sxfwd<R, L>, x_lds<R, L>());         \
         break;

@@ -9,7 +9,7 @@
 // one unfold for all of them, five barriers in all, and four to sixteen times
 // as many blocks.  The loads of the state and the history start with those of
 // the lines.  Arithmetic and order per value are k_xstep's, so a member steps
-// the same whichever kernel its launch takes (xall_log).
+// the same whichever kernel its launch takes (xtile_log).
 #pragma once
 #include "kernels.hpp"
 
@@ -215,21 +215,29 @@ __global__ __launch_bounds__(xa_threads<LOGXA>()) void k_xall(Batch bt, const cp
     }
 }
 
-// log2(XA) of the launch of nblk k_xstep blocks (2048/MM columns each), 0 for
-// k_xstep itself.  Measured on the MI355X, M4 (M6 where said), us per launch:
-//   k_xstep blocks   64^2 (8): k_xstep 50, XA 64..512 12, 12, 14, 20
-//                    M6 128^2 modes MM = NN = 128 (48): 58, XA 128..512 32, 33, 28
-//                    MM = 256, NN = 64 (32): 53, XA 256, 512 23, 28
-//                    MM = 512, NN = 64 (64): 61, XA 512 38
-//                    MM = NN = 256 (128): 57, XA 256, 512 76, 60
-//                    MM = NN = 512 (512): 148, XA 512 271
-//                    256 members of MM = NN = 64 (2048): step 899, XA 512 1067
-// Once k_xstep has half the CUs at work its longer pieces win; below, the
-// largest tile that still gives about 160 blocks does.
-template <int LOGMM> inline int xall_log(int nblk)
+// The fused x kernel of a launch of nblk full k_xstep blocks (2048/MM columns
+// each): log2 of the values of a line in a tile, 11 and 10 for k_xstep (whole and
+// half tiles), 6 to 9 for k_xall.  us per launch on the MI355X, FP64 M4 unless said:
+//   nblk   8 (MM = NN = 64):    k_xstep 50, k_xall 64..512 12, 12, 14, 20
+//         32 (256, 64):         53; 256, 512 23, 28
+//         48 (M6 128, 128):     58; 128..512 32, 33, 28
+//         64 (512, 64):         61; 512 38;  (256, 128): half tiles 43, k_xall 31
+//         96 (M6 256, 128; 512, 64; 128, 256): half tiles 44, 50, 44, k_xall 53, 67, 46
+//            (FP32: 38, 39, 36 and 38, 42, 32)
+//        128 (256, 256; 128, 512; 512, 128): whole 57, 63, 64, half 45, 45, 52; (FP32
+//            48, 48, 49 and 39, 36, 40); k_xall 512 (256, 256) 60
+//        192 (M6 256, 256):     whole 62, half 84
+//        512 (512, 512):        whole 147, half 201, k_xall 271
+//        2048 (256 members of 64, 64): a step 899, with k_xall 512 1067
+// Up to one block per CU smaller tiles win, beyond it the longer pieces do.
+// Below, k_xall takes the largest tile that still gives about 160 blocks.
+template <typename R, int LOGMM> inline int xtile_log(int nblk, int NN)
 {
-    if (LOGMM > 9 || nblk >= 128) return 0;
+    if (LOGMM > 9 || nblk > 128) return LOG_XTILE;
+    if (LOGMM >= 6 && NN >= (1 << 10) >> LOGMM && (nblk > 96 || (nblk > 64 && LOGMM >= (sizeof(R) == 8 ? 7 : 9)))) return 10;
+    if (nblk >= 128) return LOG_XTILE;
     int lx = 9;
     while (lx > 6 && lx > LOGMM && (nblk << (LOG_XTILE - lx)) < 160) lx--;
+    while (lx > LOGMM && (1 << (lx - LOGMM)) > NN) lx--; // whole tiles
     return lx;
 }

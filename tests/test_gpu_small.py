@@ -27,7 +27,7 @@ def _params(k0, mm, nn, mixed=False, theta=0.0):
 # smallest and longest rows, both bases; x tiles of 64 to 512 values, of one
 # column (MM = 512), of fewer columns than NN allows, and k_xstep's
 @pytest.mark.parametrize("k0,mm,nn", [(4, 16, 16), (6, 16, 16), (4, 16, 256), (6, 32, 128), (4, 128, 256), (6, 256, 16),
-                                      (4, 512, 16), (4, 512, 64), (6, 128, 128)])
+                                      (4, 512, 16), (4, 512, 64), (6, 128, 128), (4, 512, 128), (6, 256, 128)])
 @pytest.mark.parametrize("mixed", [False, True])
 def test_small_sizes_match_oracle(k0, mm, nn, mixed):
     p = _params(k0, mm, nn, mixed, theta=20.0)
@@ -47,12 +47,12 @@ def test_small_sizes_match_oracle(k0, mm, nn, mixed):
 
 @pytest.mark.parametrize("k0,mm,nn,mixed", [(4, 64, 64, False), (4, 64, 64, True), (4, 32, 32, False), (6, 128, 128, False),
                                             (4, 128, 32, True), (6, 16, 64, False), (4, 256, 32, False),
-                                            (4, 512, 16, True)])
+                                            (4, 512, 16, True), (6, 256, 128, False), (4, 64, 1024, True)])
 def test_members_step_alike_in_small_and_large_launches(k0, mm, nn, mixed):
-    """A single model's launches take the all-lines x kernel, those of enough
-    members of the same size k_xstep: the same bits."""
+    """A single model's launches take the all-lines x kernel or half tiles, those
+    of enough members of the same size k_xstep's whole tiles: the same bits."""
     p = _params(k0, mm, nn, mixed)
-    n = 128 // ((nn // min(nn, 2048 // mm)) * k0) + 1
+    n = 128 // ((nn // min(nn, 2048 // mm)) * k0) + 1  # more than 128 whole tiles
     ic = mw.ic_gaussian(p, 4, 0.2, 4.0)
     ens, v = mw.Ensemble([p] * n), mw.Velocity(p)
     for i in range(n):
