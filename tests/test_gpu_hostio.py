@@ -28,8 +28,9 @@ def _round_trip(k0, mm, nn, mixed, seed):
     v.close()
 
 
-# 16: a state of 40 KB; (6, 64, 64): the field just over a chunk (4 MB); (4, 256, 256): a state of four chunks
-@pytest.mark.parametrize("k0,mm,nn", [(4, 16, 16), (6, 16, 128), (6, 64, 64), (4, 256, 256), (6, 512, 32)])
+# (4, 16, 16): a state of 55 KB; (4, 256, 256): two chunks of 8 MB; (6, 256, 512): more than the four
+# chunks of a handle's staging
+@pytest.mark.parametrize("k0,mm,nn", [(4, 16, 16), (6, 16, 128), (6, 64, 64), (4, 256, 256), (6, 512, 32), (6, 256, 512)])
 @pytest.mark.parametrize("mixed", [False, True])
 def test_state_and_history_round_trip(k0, mm, nn, mixed):
     _round_trip(k0, mm, nn, mixed, mm + nn)
