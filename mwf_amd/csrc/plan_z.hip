@@ -151,9 +151,11 @@ template <typename R, int K0> void pick_z(int ln, Plan& p)
         p.zphys = launch_zphys<R, K0, 10>;
         p.zfwdp = launch_zfwdp<R, 10>;
         // the flux z kernel holds all three phases of a 3072-point row at
-        // 1024 threads (4 waves per SIMD) in FP32 only; in FP64 three blocks
-        // share the row
-        if constexpr (std::is_same<R, float>::value) p.zc = launch_zc<R, K0, 10, 4>;
+        // 1024 threads (4 waves per SIMD) in FP32 only (with two buffers, a
+        // barrier per batch fewer: M6 2048^2 625 -> 593 us; larger batches of 12
+        // or 18 sequences in one buffer, 753 and 1062); in FP64 three blocks share
+        // the row
+        if constexpr (std::is_same<R, float>::value) p.zc = launch_zc<R, K0, 10, 2>;
         else {
             p.zc = launch_zc3<R, K0, 10>;
             p.zc_split = true;
@@ -189,7 +191,7 @@ template <typename R, int K0> void prepare_z(int ln)
         set_lds(k_zphys<R, K0, 10>, zphys_lds<R, 10>());
         set_lds(k_zfwd_phys<R, 10>, zfp_lds<R, 10>());
         if constexpr (std::is_same<R, float>::value)
-            set_lds(k_zc<R, K0, 10, ZC_ZP, 4, false>, zc_lds_bytes<R, 10, ZC_ZP, false>());
+            set_lds(k_zc<R, K0, 10, ZC_ZP, zc_waves<R, 2>(), true>, zc_lds_bytes<R, 10, ZC_ZP, true>());
         else set_lds(k_zc3<R, K0, 10, ZC_ZP>, zc_lds_bytes<R, 10, ZC_ZP, false>());
         break;
     default: break;
