@@ -38,15 +38,15 @@ TURB_CT = 1e-2
 
 
 def step_bytes(mw, p):
-    """Algorithmic HBM bytes of one step of one member (the two-pass model):
-    state c read and written (complex FP64), AB2 history read and written (in
-    the transform precision), and one HBM round trip of the x-physical /
-    z-spectral intermediates: 3 KK lines of P x NN complex values each way
+    """Algorithmic HBM bytes of one step of one member in the flux form: state c
+    read and written (complex FP64), AB2 history read and written (in the
+    transform precision), and one HBM round trip of the x-physical / z-spectral
+    intermediates: KK lines of U and 4 K0 - 2 of NL, of P x NN complex values
     (written once, read once)."""
     d = mw.dims(p)
     si = 8 if p.precision == mw.MWF_MIXED else 16
     mpt = d["K"] * d["M"] * p.nn
-    return 2 * 16 * mpt + 2 * si * mpt + 2 * 3 * d["KK"] * d["P"] * p.nn * si
+    return 2 * 16 * mpt + 2 * si * mpt + 2 * (d["KK"] + 4 * p.k0 - 2) * d["P"] * p.nn * si
 
 
 def run_gpu(mw, precision, steps, warmup, ic, workload=WORKLOAD, event_steps=200):

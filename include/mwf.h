@@ -173,7 +173,7 @@ int mwf_autotune(int32_t mode);
  * (conservative) form of vel_nonlinear's products: the same projected
  * (u.grad)u, with d/dx, d/dz taken in spectral space and d/dy moved onto the
  * wall-normal bases, equal to the advective form up to rounding; bit 4 (with
- * bit 3) = its z kernel compiled for two waves per SIMD instead of four;
+ * bit 3) = its z kernel with two LDS buffers, a barrier per batch fewer;
  * bit 5 (advective form, NN = 1024; implies bit 1 in the mixed form) = the
  * phase-sequential z kernel with the three fold phases of an x-row in three
  * blocks, each writing its own NL partial, which the x kernel sums. */

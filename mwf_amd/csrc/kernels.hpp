@@ -1,9 +1,11 @@
 // kernels.hpp -- the per-step kernels of the Model Waleffe Flow timestepper.
 //
-// One step (program/velocity.f90:21-41) is three launches:
+// One step (program/velocity.f90:21-41) of the advective form is three launches:
 //   k_xinv : state c  -> U   mpt2spec + laminar + d/dx, padded inverse x-DFT
 //   k_z    : U        -> NL  z c2r of u, du/dx, du/dz; udotgradu; z r2c
 //   k_xfwd : NL, c    -> c   forward x-DFT, spec2mpt, AB2 + implicit update
+// the last and the next step's first fused in k_xstep.  The flux form
+// (zflux.hpp, zbatch.hpp, xall.hpp) has its own lines of U and NL.
 //
 // Device layouts (complex values interleaved):
 //   c        double2 [NN][K][ldM]      m in the reference order (m<0 at M+m)

@@ -160,16 +160,16 @@ template <typename T> static int dev_upload(T** d, const T* h, size_t n)
 // (program/transform.fftw5.f90:33-59).  Mode 0 (default): the rule-based plan
 // (SizeClass::rule).  Mode 1: each
 // new size class times its candidate plans on its own buffers (zero state,
-// best of 3 interleaved rounds of 5 steps) and keeps the fastest; the choice
+// the best of several interleaved rounds of steps) and keeps the fastest; the choice
 // is cached per (precision, K0, MM, NN) for the process, so every handle and
-// ensemble class of one size runs the same kernels.  Modes 2..9 force choice
+// ensemble class of one size runs the same kernels.  Modes 2..65 force choice
 // mode - 2 (where the alternative exists), for tests and plan comparisons.
 // Choice bits: 1 = phase-sequential z kernel (k_zb) instead of k_z, 2 =
 // x-inverse + x-forward instead of the fused x kernel, 4 = two-points-per-
 // thread z kernel (k_z2; takes precedence over bit 1), 8 = flux form of the
 // nonlinear term (k_zc and the flux x kernels; takes precedence over bits 1
-// and 4, where it exists), 16 = with bit 8, the flux z kernel compiled for
-// 2 waves per SIMD (no spills) instead of 4 (two blocks per CU), 32 = at
+// and 4, where it exists), 16 = with bit 8, the flux z kernel with two LDS
+// buffers and a barrier per batch fewer (in FP64 one block per CU instead of two), 32 = at
 // NN = 1024 in the advective form, k_zb with the fold phases of a row in
 // three blocks and three NL partials (with the split x kernels).
 // ---------------------------------------------------------------------------

@@ -32,11 +32,11 @@ struct Plan {
     // (bt.nl_part), summed by the split x kernels
     hipError_t (*zf_ph3)(const Batch&, int, const Geo&, hipStream_t, const void*, void*, const void*,
                          const void*) = nullptr;
-    // flux form (zflux.hpp): z kernel and the x kernels that read its B/A lines
+    // flux form (zflux.hpp): z kernel and the x kernels that read its lines (dev_line)
     // and write U without x-derivative lines
     hipError_t (*zc)(const Batch&, int, const Geo&, hipStream_t, const void*, void*, const void*, const void*) = nullptr;
     hipError_t (*zc_alt)(const Batch&, int, const Geo&, hipStream_t, const void*, void*, const void*,
-                         const void*) = nullptr; // the flux z kernel at 2 waves per SIMD instead of 4
+                         const void*) = nullptr; // the flux z kernel with two buffers
     bool zc_split = false; // zc writes dev_lines_split(K0) lines
     bool zc_batch = false; // zc takes a whole x-row in one batch (zbatch.hpp)
     hipError_t (*xinv_f)(const Batch&, int, const Geo&, hipStream_t, const double2*, void*, double*, const void*,

@@ -23,7 +23,8 @@
 // 22.  The form with one line to be differentiated in x and one for the rest per
 // spec slot has 21 rows and 22 lines (33 and 34), so 36 % of NL's bytes and of
 // the forward x transforms are saved: at M4 1024^2 k_zc 157 -> 141 us and
-// k_xstep 192 -> 149 us in FP64, 79 -> 72 and 121 -> 101 us in FP32.
+// k_xstep 192 -> 149 us in FP64, 79 -> 72 and 121 -> 101 us in FP32 (133, 147, 68.5
+// and 100 us with the later changes noted below and in kernels.hpp).
 // Of the equivalent pairs of lines this one keeps the largest products, uu, at
 // the weights a^2 and a g they have in the plain form (E and g (ww - uu) - i ak vw
 // would add a g^2), which the rounding of the FP32 form follows.
@@ -201,7 +202,7 @@ __device__ __forceinline__ void zc_pass(const Geo& g, int xt, const cplx_t<R>* _
     auto buf_of = [&](int k) { return (PP && (k & 1)) ? bufB : bufA; };
     // transforms of the first S sequences of b, in place, natural order in
     // and out; ends with a block barrier.  Lane-group transforms where their
-    // registers fit (NN <= 512, and FP32 or the two-wave form); otherwise
+    // registers fit (NN <= 512, and FP32 or the two-buffer form); otherwise
     // Stockham passes over the whole block (ip_fft, a barrier per half-pass).
     constexpr bool WAVE = zc_wave<R, LOGNN, PP>();
     auto transform = [&](auto sign, int S, CT* b, int t) {
@@ -384,8 +385,8 @@ __device__ __forceinline__ void zc_pass(const Geo& g, int xt, const cplx_t<R>* _
         // forward sequences: pair q, phase b at 3 q + b.  With an odd number
         // of rows the last pair holds one row, whose three phases take two
         // sequences (phases 0 and 1 as the real and imaginary parts of the
-        // first, phase 2 in the second): M4's 21 rows fill 4 batches of 8
-        // instead of 5
+        // first, phase 2 in the second): M4's 17 rows are 26 sequences
+        // instead of 27 (FP64: 4 batches instead of 5)
         constexpr bool LONE = NR % 2 == 1;
         constexpr int QL = NPO - 1;                  // the last pair
         constexpr int NSF = 3 * NPO - (LONE ? 1 : 0);
