@@ -282,7 +282,7 @@ class Velocity:
     def plan_info(self):
         """Plan bits: PLAN_ZB (phase-sequential z kernel), PLAN_SPLIT_X (separate x kernels),
         PLAN_Z2 (two-points-per-thread z kernel), PLAN_FLUX (flux form), PLAN_FLUX_W2 (its
-        two-wave z kernel), PLAN_ZB_SPLIT (the fold phases of a row in three blocks)."""
+        z kernel with two buffers), PLAN_ZB_SPLIT (the fold phases of a row in three blocks)."""
         ch = ctypes.c_int32()
         _check(lib().mwf_plan_info(self._h, ctypes.byref(ch)))
         return ch.value
