@@ -6,6 +6,8 @@
 #include <type_traits>
 #include <utility>
 
+#include "fluxline.hpp"
+
 template <typename R> struct cplx_of;
 template <> struct cplx_of<double> { using type = double2; };
 template <> struct cplx_of<float> { using type = float2; };
@@ -141,12 +143,3 @@ __device__ __forceinline__ size_t nidx(const Geo& g, int x, int slot, int n)
 // wall-normal derivative table ad_k1, ad_k2 (program/variables.f90:528-531)
 __device__ __forceinline__ double ak1_of(int k, double beta) { return ((k & 1) ? -1.0 : 1.0) * k * beta; }
 __device__ __forceinline__ double ak2_of(int k, double beta) { return -k * k * beta * beta; }
-
-// Lines of NL in the flux form (zflux.hpp): per wall-normal index k >= 1 uw,
-// F, uv, E, for k = 0 uw and F.
-enum { DEV_UW, DEV_F, DEV_UV, DEV_E };
-__host__ __device__ constexpr int dev_line(int k) { return k == 0 ? 0 : 4 * k - 2; }
-__host__ __device__ constexpr int dev_lines(int K0) { return 4 * K0 - 2; }
-// with the vw share of E_k on a line of its own, dev_lines + k - 1 (FP64 rows of
-// 1024 points; Geo::NLL tells the x kernels)
-__host__ __device__ constexpr int dev_lines_split(int K0) { return 5 * K0 - 3; }

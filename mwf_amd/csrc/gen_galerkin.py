@@ -41,7 +41,7 @@ spectral space:
 
 The z kernel of this form needs only the rows of dev_rows (five per i >= 1): the
 step takes the nonlinear term as its psi and phi parts, and in those the
-products' trace drops out (zflux.hpp has the algebra).
+products' trace drops out (fluxline.hpp has the algebra).
 
 Run:  python mwf_amd/csrc/gen_galerkin.py   (rewrites galerkin_gen.hpp and flux_gen.hpp)
 """

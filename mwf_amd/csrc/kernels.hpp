@@ -1129,39 +1129,24 @@ __device__ __forceinline__ void s2m_finish(int k, int mi, int n, double2 u, doub
     }
 }
 
-// Flux form: the share of line type li (uw, F, uv, E of wall-normal index k,
-// zflux.hpp; not yet scaled, dev_scale) in psi_k and phi_k of the nonlinear term
-// at one (m, n), from the line's forward x transform X; rak = 1/ak1, for k = 0
-// -1 (F_0 has the multiplier a).  At (0,0), where every multiplier vanishes, the
-// mean-mode rows of var_spec2mpt apply instead: psi = -N_u = -ak uv, phi = -N_w =
-// i F / ak.
-__device__ __forceinline__ void dev_term(int li, bool mean, double2 X, double am1, double an1, double ak1, double rak,
-                                         double2& psi, double2& phi)
+// Flux form: the share of line type li (fluxline.hpp; not yet scaled, dev_scale)
+// in psi_k and phi_k of the nonlinear term at one (m, n), from the line's forward
+// x transform X.  At (0,0), where every weight vanishes, the mean-mode rows of
+// var_spec2mpt apply instead: psi = -N_u = -ak uv, phi = -N_w = -ak vw = i B.
+__device__ __forceinline__ void dev_term(int li, bool mean, double2 X, double am1, double an1, double ak1, double2& psi,
+                                         double2& phi)
 {
 #pragma clang fp contract(off)
     if (li == DEV_UV) X = double2{-X.y, X.x}; // i uv
-    const double a2 = am1 * am1, g2 = an1 * an1;
     double cp, cq;
-    if (li == DEV_UW) {
-        cp = a2 - g2;
-        cq = -2.0 * ak1 * (am1 * an1);
-    } else if (li == DEV_F) {
-        cp = -(am1 * rak);
-        cq = an1;
-    } else if (li == DEV_UV) {
-        cp = an1 * ak1;
-        cq = am1 * (ak1 * ak1 - (a2 + g2));
-    } else {
-        cp = am1 * an1 * rak;
-        cq = a2;
-    }
+    dev_weights(li, am1, an1, ak1, cp, cq);
     psi.x = __builtin_fma(cp, X.x, psi.x);
     psi.y = __builtin_fma(cp, X.y, psi.y);
     phi.x = __builtin_fma(cq, X.x, phi.x);
     phi.y = __builtin_fma(cq, X.y, phi.y);
     if (mean) {
         if (li == DEV_UV) psi = double2{-(ak1 * X.y), ak1 * X.x}; // -ak uv, X = i uv
-        if (li == DEV_F) phi = double2{-(X.y * rak), X.x * rak};
+        if (li == DEV_F) phi = double2{-X.y, X.x};
     }
 }
 
@@ -1279,7 +1264,7 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
     const int k = blockIdx.y;
     const int tid = threadIdx.x;
     const int nitems = NT * MM;
-    const double ak1 = ak1_of(k, g.beta), rak = k == 0 ? -1.0 : 1.0 / ak1;
+    const double ak1 = ak1_of(k, g.beta);
 
     // flux form: psi[] and phi[] sum the lines' shares; otherwise psi[] holds
     // u_k until w_k arrives, phi[] holds v_k (am2+an2) until then
@@ -1303,7 +1288,7 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
             const int a = x / 3, b = x - 3 * a;
             const int po = pan_at(g, g.lgNT, it);
             CT v = pan[po];
-            if (FLUX && li == DEV_E && g.NLL > dev_lines(g.K0)) // the vw share of E
+            if (FLUX && li == DEV_E && g.NLL > dev_lines(g.K0)) // its vw and ww shares
                 v = cadd(v, pan[po + evw]);
             if (!FLUX && bt.nl_part) { // the z pass's three fold-phase partials: ((P0 + P1) + P2) / (PQ)
                 const CT v1 = pan[po + bt.nl_part], v2 = pan[po + 2 * bt.nl_part];
@@ -1332,7 +1317,7 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
                 zwave(g, n, an1, an2);
                 const double2 X = X0;
                 if constexpr (FLUX) {
-                    dev_term(li, mi == 0 && n == 0, X, am1, an1, ak1, rak, psi[q][h], phi[q][h]);
+                    dev_term(li, mi == 0 && n == 0, X, am1, an1, ak1, psi[q][h], phi[q][h]);
                     continue;
                 }
                 // var_spec2mpt (program/variables.f90:440-480)
@@ -1517,7 +1502,7 @@ __global__ __launch_bounds__(xs_of<LXT>(), 3) void k_xstep(Batch bt, const cplx_
         rb = reg + (t0 * 3 + b0) * MM;
         pa = pidx(a0) ^ xsw<R>(t0, b0);
     };
-    const double ak1 = ak1_of(k, g.beta), rak = k == 0 ? -1.0 : 1.0 / ak1;
+    const double ak1 = ak1_of(k, g.beta);
     const double ak2 = ak2_of(k, g.beta);
 
     // flux form: psi[] and phi[] sum the lines' shares; otherwise psi[] holds
@@ -1584,7 +1569,7 @@ __global__ __launch_bounds__(xs_of<LXT>(), 3) void k_xstep(Batch bt, const cplx_
                 // NL element, or the sum ((P0 + P1) + P2) / (PQ) of the three
                 // fold-phase partials of the phase-split z kernel
                 const size_t nlp = FLUX ? 0 : bt.nl_part;
-                // flux form: where E's vw share has a line of its own, add it
+                // flux form: where DEV_E's vw and ww shares have a line of their own, add it
                 const bool esum = FLUX && li == DEV_E && g.NLL > dev_lines(g.K0);
                 const ptrdiff_t evw = (ptrdiff_t)(dev_lines(g.K0) + k - 1 - (dev_line(k) + DEV_E)) * g.P * g.NTs;
                 auto nl_at = [&](const CT* p) {
@@ -1660,7 +1645,7 @@ __global__ __launch_bounds__(xs_of<LXT>(), 3) void k_xstep(Batch bt, const cplx_
                     xwave(g, mi, am1, am2);
                     zwave(g, n, an1, an2);
                     if constexpr (FLUX) {
-                        dev_term(li, mi == 0 && n == 0, X, am1, an1, ak1, rak, psi[q][h], phi[q][h]);
+                        dev_term(li, mi == 0 && n == 0, X, am1, an1, ak1, psi[q][h], phi[q][h]);
                         continue;
                     }
                     if (li == 0) {

@@ -184,14 +184,13 @@ __global__ __launch_bounds__((zs_threads<K0, LOGNN>())) void k_zs(Batch bt, cons
         };
         CT* nlr = NL + ((((size_t)(n >> g.lgNS) * dev_lines(K0) + dev_line(k)) * g.P + x) << g.lgNS) + (n & (g.NTs - 1));
         const size_t nls = (size_t)g.P << g.lgNS;
-        const double gd = g.gamma * n, ak = ak1_of(k, g.beta);
-        const R gn = (R)gd;
+        const double gn = g.gamma * n;
         CT uw;
         if (k == 0) {
             CT d;
             pair(buf, uw, d);
             st_piece(nlr + DEV_UW * nls, uw, wide);
-            st_piece(nlr + DEV_F * nls, cscale(d, gn), wide);
+            st_piece(nlr + DEV_F * nls, cscale(d, (R)-gn), wide);
             continue;
         }
         const CT* sk = buf + (3 + 8 * (k - 1)) * LPZ;
@@ -204,8 +203,9 @@ __global__ __launch_bounds__((zs_threads<K0, LOGNN>())) void k_zs(Batch bt, cons
         vw = cadd(vw, cmul(a, w1));
         split(sk + 7 * LPZ, a, c);
         vw = cadd(vw, cmul(a, w2));
-        const R akr = (R)ak, akg = (R)(ak * gd), f5 = (R)(ak * ak - gd * gd);
-        st_piece(nlr + DEV_F * nls, CT{akg * vvww.x - f5 * vw.y, akg * vvww.y + f5 * vw.x}, wide);
-        st_piece(nlr + DEV_E * nls, CT{akr * vvuu.x + gn * vw.y, akr * vvuu.y - gn * vw.x}, wide);
+        const DevMul<R> m = dev_mul<R>(gn, ak1_of(k, g.beta));
+        if (m.far) vvuu = csub(vvuu, vvww); // ww - uu
+        st_piece(nlr + DEV_F * nls, CT{m.f * vvww.x - m.h * vw.y, m.f * vvww.y + m.h * vw.x}, wide);
+        st_piece(nlr + DEV_E * nls, CT{vvuu.x + m.e * vw.y, vvuu.y - m.e * vw.x}, wide);
     }
 }

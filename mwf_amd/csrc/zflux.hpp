@@ -7,27 +7,16 @@
 // v_k, w_k; no x- or z-derivatives).  The step needs the nonlinear term only as
 // its psi and phi parts (var_spec2mpt), and of the six projected products
 // uu, uw, ww, uv, vw, vv of a wall-normal index k these take the trace-free
-// part alone (the trace is a pressure gradient).  With a = alpha m,
-// g = gamma n, ak = ak1(k):
-//
-//   E_k = ak (vv_k - uu_k) - i g vw_k
-//   F_k = ak g (vv_k - ww_k) + i (ak^2 - g^2) vw_k
-//   psi_k = (a^2 - g^2) uw_k + i g ak uv_k + (a g / ak) E_k - (a / ak) F_k
-//   phi_k = i a (ak^2 - a^2 - g^2) uv_k - 2 ak a g uw_k + a^2 E_k + g F_k
-//   psi_0 = (a^2 - g^2) uw_0 + a F_0,  F_0 = g (ww_0 - uu_0)
-//
-// so five real rows per k >= 1 (uv, uw, vv - uu, vw, vv - ww; two for k = 0) are
-// transformed forward, and four lines per k >= 1 (uw, F, uv, E; two for k = 0)
-// cross to the x kernel, which applies the powers of a and the scale 1/(2 PQ)
-// (Dev below, and dev_term in kernels.hpp): M4 17 rows and 14 lines, M6 27 and
-// 22.  The form with one line to be differentiated in x and one for the rest per
-// spec slot has 21 rows and 22 lines (33 and 34), so 36 % of NL's bytes and of
-// the forward x transforms are saved: at M4 1024^2 k_zc 157 -> 141 us and
-// k_xstep 192 -> 149 us in FP64, 79 -> 72 and 121 -> 101 us in FP32 (133, 147, 68.5
-// and 100 us with the later changes noted below and in kernels.hpp).
-// Of the equivalent pairs of lines this one keeps the largest products, uu, at
-// the weights a^2 and a g they have in the plain form (E and g (ww - uu) - i ak vw
-// would add a g^2), which the rounding of the FP32 form follows.
+// part alone (the trace is a pressure gradient): five real rows per k >= 1 (uv,
+// uw, vv - uu, vw, vv - ww; two for k = 0) are transformed forward, and four lines
+// per k >= 1 (two for k = 0; fluxline.hpp has them and their algebra) cross to the
+// x kernel, which applies the powers of a and the scale 1/(2 PQ) (Dev below, and
+// dev_term in kernels.hpp): M4 17 rows and 14 lines, M6 27 and 22.  The form with
+// one line to be differentiated in x and one for the rest per spec slot has 21 rows
+// and 22 lines (33 and 34), so 36 % of NL's bytes and of the forward x transforms
+// are saved: at M4 1024^2 k_zc 157 -> 141 us and k_xstep 192 -> 149 us in FP64, 79
+// -> 72 and 121 -> 101 us in FP32 (134, 148, 69 and 101 us with the later changes
+// noted below and in kernels.hpp and the line pair chosen per n).
 //
 // Block: T = max(512, NN) threads, XB = T/NN x-rows; thread (xl, r) owns the
 // points z = 3r + b, b = 0..2, of row xl, and the output index n = r of that
@@ -59,8 +48,8 @@
 // PART 0 is the whole pass.  PART 1, 2, 3 take the rows that need two of the
 // three components only (u w: uw and ww_0 - uu_0; u v: uv, vv - uu; v w: vw,
 // vv - ww), for rows so long that one block's registers do not hold all the base
-// values of its points; the vw share of E_k then goes to a line of its own, dev_lines +
-// k - 1, which the x kernel adds.
+// values of its points; the vw and ww shares of line DEV_E then go to a line of their
+// own, dev_lines + k - 1, which the x kernel adds.
 template <int K0_, int PART = 0> struct Dev {
     static constexpr int K0 = K0_;
     // base lines, and the spec slot of base line i
@@ -82,21 +71,21 @@ template <int K0_, int PART = 0> struct Dev {
         if (PART == 1) return q < 2 ? q : 2 + 5 * (q - 2) + UW;
         return 2 + 5 * (q / 2) + (PART == 2 ? (q & 1 ? VVUU : UV) : (q & 1 ? VVWW : VW));
     }
-    // uses of row r: line, kind (0: row, 1: ak row, 2: g row, 3: -i g row, 4: ak g row, 5: i (ak^2 - g^2) row)
-    __host__ __device__ static constexpr int nuse(int r) { return type(r) == VW ? 2 : 1; }
+    // uses of row r: line, kind
+    enum { ROW, NEG_G, VW_E, VW_F, WW_E, WW_F }; // row, -g row, and the multiples of DevMul
+    __host__ __device__ static constexpr int nuse(int r) { return type(r) == VW || type(r) == VVWW ? 2 : 1; }
     __host__ __device__ static constexpr int use_line(int r, int u)
     {
         const int t = type(r);
-        if (PART != 0 && t == VW && u == 0) return dev_lines(K0) + k(r) - 1;
-        return dev_line(k(r)) + (t == UW ? DEV_UW : t == UV ? DEV_UV : t == VVUU || (t == VW && u == 0) ? DEV_E : DEV_F);
+        const bool e = (t == VW || t == VVWW) && u == 0; // the vw or ww share of DEV_E
+        if (PART != 0 && e) return dev_lines(K0) + k(r) - 1;
+        return dev_line(k(r)) + (t == UW ? DEV_UW : t == UV ? DEV_UV : t == VVUU || e ? DEV_E : DEV_F);
     }
     __host__ __device__ static constexpr int use_kind(int r, int u)
     {
         const int t = type(r);
-        return t == VVUU ? 1 : t == WWUU ? 2 : t == VW ? (u == 0 ? 3 : 5) : t == VVWW ? 4 : 0;
+        return t == WWUU ? NEG_G : t == VW ? (u == 0 ? VW_E : VW_F) : t == VVWW ? (u == 0 ? WW_E : WW_F) : ROW;
     }
-    // ak1(k) / beta = (-1)^k k (program/variables.f90:528-529)
-    __host__ __device__ static constexpr int sign(int r) { return (k(r) & 1) ? -k(r) : k(r); }
     // forward positions of the first and the last row of line L
     __host__ __device__ static constexpr int first(int L)
     {
@@ -336,9 +325,8 @@ __device__ __forceinline__ void zc_pass(const Geo& g, int xt, const cplx_t<R>* _
     });
 
     // ---- products, forward z transforms (r2c, -1), line assembly ----
-    const R gn = (R)(g.gamma * r);       // gamma n at the thread's output n = r
-    const R beta = (R)g.beta, bg = (R)(g.beta * (g.gamma * r));
-    const R b2 = (R)(g.beta * g.beta), g2 = (R)((g.gamma * r) * (g.gamma * r));
+    const double gn = g.gamma * r, rgn = 1.0 / gn; // gamma n at the thread's output n = r
+    const double rbeta = 1.0 / g.beta;
     const R lu = (R)g.cth, lw = (R)g.sth; // laminar u_1, w_1
     if constexpr (HT) {
         tf[0] = cconj(twQl[r]);
@@ -360,15 +348,15 @@ __device__ __forceinline__ void zc_pass(const Geo& g, int xt, const cplx_t<R>* _
                 static_for<0, FX::nuse(row)>([&](auto ui) {
                     constexpr int u = decltype(ui)::value;
                     constexpr int L = FX::use_line(row, u), kind = FX::use_kind(row, u);
-                    constexpr int sg = FX::sign(row);
+                    constexpr int k = FX::k(row);
                     CT term = xs;
-                    if constexpr (kind == 1) term = cscale(xs, (R)sg * beta);
-                    else if constexpr (kind == 2) term = cscale(xs, gn);
-                    else if constexpr (kind == 3) term = CT{xs.y * gn, -(xs.x * gn)};
-                    else if constexpr (kind == 4) term = cscale(xs, (R)sg * bg);
-                    else if constexpr (kind == 5) {
-                        const R f = (R)(sg * sg) * b2 - g2;
-                        term = CT{-(xs.y * f), xs.x * f};
+                    if constexpr (kind == FX::NEG_G) term = cscale(xs, (R)-gn);
+                    else if constexpr (kind != FX::ROW) {
+                        const DevMul<R> m = dev_mul<R>(gn, rgn, ak1_of(k, g.beta), (k & 1 ? -1.0 : 1.0) / k * rbeta);
+                        if constexpr (kind == FX::VW_E) term = CT{xs.y * m.e, -(xs.x * m.e)};
+                        else if constexpr (kind == FX::VW_F) term = CT{-(xs.y * m.h), xs.x * m.h};
+                        else if constexpr (kind == FX::WW_E) term = m.far ? CT{-xs.x, -xs.y} : CT{(R)0, (R)0};
+                        else term = cscale(xs, m.f);
                     }
                     if constexpr (FX::first(L) == q) acc[L] = term;
                     else acc[L] = cadd(acc[L], term);
