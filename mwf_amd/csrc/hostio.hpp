@@ -64,6 +64,14 @@ __global__ __launch_bounds__(256) void k_planes_in(const double* __restrict__ re
     }
 }
 
+// words of 8 bytes between device memory and a pinned chunk
+static __global__ __launch_bounds__(256) void k_words(const unsigned long long* __restrict__ src, unsigned long long* __restrict__ dst,
+                                                      unsigned n)
+{
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
 // A few copy threads, shared by every handle of the process and gone with the
 // last one.  run() is one user's at a time; another caller meanwhile does its
 // own work alone.
@@ -165,11 +173,16 @@ private:
 };
 
 // Pinned staging of one handle: chunks, each with the event of its last copy.
-// A transfer that fits one chunk is one copy and one wait (each costs some 20 us
-// whatever its size); longer ones run through all the chunks.
+// Transfers of up to DIRECT bytes are read or written by kernels in the first chunk
+// itself, over the bus: a DMA after a kernel costs some 10 us more than the kernel
+// alone, and now and then 100 (get_state of M4 32^2 modes, 54 KB, 28 us and at times
+// 132 with the DMA, 18 without; 64^2, 220 KB, 35 and 24; 128^2, 889 KB, 64 and 53;
+// from 1.4 MB on the two are alike).  A transfer that fits one chunk is one copy and
+// one wait; longer ones run through all the chunks.
 struct HostStage {
     static constexpr size_t CHUNK = 8 << 20; // M6 2048^2 get_state: 4 MB chunks 14 ms, 8 and 16 MB 9.4
     static constexpr int NSLOT = 4;
+    static constexpr size_t DIRECT = 1 << 20;
     char* buf = nullptr;
     size_t chunk = 0;
     int nslot = 0;
@@ -192,9 +205,36 @@ struct HostStage {
         if (buf) (void)hipHostFree(buf);
         *this = HostStage{};
     }
+    // a transfer that kernels make themselves, to or from the first chunk
+    bool direct(size_t bytes) const { return bytes <= DIRECT && bytes <= chunk; }
+    hipError_t words(hipStream_t st, const void* src, void* dst, size_t bytes)
+    {
+        const unsigned n = (unsigned)(bytes / 8);
+        hipLaunchKernelGGL(k_words, dim3((n + 255) / 256), dim3(256), 0, st, (const unsigned long long*)src,
+                           (unsigned long long*)dst, n);
+        return hipGetLastError();
+    }
+    // the first chunk to or from the host's arrays
+    hipError_t drain(hipStream_t st, size_t bytes, void* dst0, size_t n0, void* dst1)
+    {
+        const hipError_t e = hipStreamSynchronize(st);
+        if (e != hipSuccess) return e;
+        pool->copy(dst0, buf, n0);
+        if (bytes > n0) pool->copy(dst1, buf + n0, bytes - n0);
+        return e;
+    }
+    void fill(size_t bytes, const void* src0, size_t n0, const void* src1)
+    {
+        pool->copy(buf, src0, n0);
+        if (bytes > n0) pool->copy(buf + n0, src1, bytes - n0);
+    }
     // device -> host, complete on return; the source's first n0 bytes go to dst0, the rest to dst1
     hipError_t d2h(hipStream_t st, const void* src, size_t bytes, void* dst0, size_t n0, void* dst1)
     {
+        if (direct(bytes)) {
+            const hipError_t e = words(st, src, buf, bytes);
+            return e != hipSuccess ? e : drain(st, bytes, dst0, n0, dst1);
+        }
         const size_t nc = (bytes + chunk - 1) / chunk;
         auto len = [&](size_t c) { return std::min(chunk, bytes - c * chunk); };
         auto slot = [&](size_t c) { return buf + (c % nslot) * chunk; };
@@ -218,6 +258,11 @@ struct HostStage {
     // host -> device, the sources read on return; n0 bytes from src0, the rest from src1
     hipError_t h2d(hipStream_t st, void* dst, size_t bytes, const void* src0, size_t n0, const void* src1)
     {
+        if (direct(bytes)) {
+            fill(bytes, src0, n0, src1);
+            const hipError_t e = words(st, buf, dst, bytes);
+            return e != hipSuccess ? e : hipStreamSynchronize(st);
+        }
         const size_t nc = (bytes + chunk - 1) / chunk;
         hipError_t e = hipSuccess;
         for (size_t c = 0; c < nc && e == hipSuccess; c++) {
@@ -240,20 +285,28 @@ template <typename CT>
 inline hipError_t planes_d2h(HostStage& hs, hipStream_t st, const Geo& g, int slots, const CT* rows, double* scratch,
                              double* re, double* im)
 {
-    const size_t n = (size_t)g.NN * g.M * slots;
+    const size_t n = (size_t)g.NN * g.M * slots, bytes = 2 * sizeof(double) * n;
+    const bool direct = hs.direct(bytes);
+    double* pl = direct ? reinterpret_cast<double*>(hs.buf) : scratch;
     hipLaunchKernelGGL(k_planes_out<CT>, dim3((g.M + PLT - 1) / PLT, g.NN), dim3(256), slots * (PLT + 1) * sizeof(CT), st,
-                       rows, slots, g.M, g.ldM, scratch, scratch + n);
+                       rows, slots, g.M, g.ldM, pl, pl + n);
     hipError_t e = hipGetLastError();
-    return e != hipSuccess ? e : hs.d2h(st, scratch, 2 * sizeof(double) * n, re, sizeof(double) * n, im);
+    if (e != hipSuccess) return e;
+    return direct ? hs.drain(st, bytes, re, bytes / 2, im) : hs.d2h(st, scratch, bytes, re, bytes / 2, im);
 }
 template <typename CT>
 inline hipError_t planes_h2d(HostStage& hs, hipStream_t st, const Geo& g, int slots, const double* re, const double* im,
                              double* scratch, CT* rows)
 {
-    const size_t n = (size_t)g.NN * g.M * slots;
-    const hipError_t e = hs.h2d(st, scratch, 2 * sizeof(double) * n, re, sizeof(double) * n, im);
+    const size_t n = (size_t)g.NN * g.M * slots, bytes = 2 * sizeof(double) * n;
+    const bool direct = hs.direct(bytes);
+    hipError_t e = hipSuccess;
+    if (direct) hs.fill(bytes, re, bytes / 2, im);
+    else e = hs.h2d(st, scratch, bytes, re, bytes / 2, im);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_planes_in<CT>, dim3((g.ldM + PLT - 1) / PLT, g.NN), dim3(256), slots * (PLT + 1) * sizeof(CT), st,
-                       scratch, scratch + n, slots, g.M, g.ldM, rows);
-    return hipGetLastError();
+    const double* pl = direct ? reinterpret_cast<const double*>(hs.buf) : scratch;
+    hipLaunchKernelGGL(k_planes_in<CT>, dim3((g.ldM + PLT - 1) / PLT, g.NN), dim3(256), slots * (PLT + 1) * sizeof(CT), st, pl,
+                       pl + n, slots, g.M, g.ldM, rows);
+    e = hipGetLastError();
+    return e == hipSuccess && direct ? hipStreamSynchronize(st) : e; // the chunk is free for the next transfer
 }
