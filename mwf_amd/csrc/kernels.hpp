@@ -1379,8 +1379,8 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
 // ---------------------------------------------------------------------------
 // Fused x kernel of one step: forward x transform of NL, spec2mpt, AB2 and
 // implicit update of c and onl, then the inverse x transform of the updated
-// state for the next step's z kernel (mpt2spec + laminar + d/dx), so c is read
-// once per step.  Block (n-tile, y-mode k), 768 threads: each group of MM/8
+// state for the next step's z kernel (mpt2spec; in the advective form + laminar
+// and d/dx), so c is read once per step.  Block (n-tile, y-mode k), 768 threads: each group of MM/8
 // lanes owns one of the 3*NT sequences (t, b), 8 points per lane, and
 // transforms it with group_fft (for MM <= 512 with no block barrier inside a
 // transform); items (t, r), up to three per thread, hold psi_k / phi_k at m = r
@@ -1466,7 +1466,6 @@ __global__ __launch_bounds__(xs_of<LXT>(), 3) void k_xstep(Batch bt, const cplx_
     // tile's sequences straight from the staged panel (element a of sequence
     // (t, b) at panel row 3a + b, column t), with no copy into the transform
     // layout and no barrier between (k_xstep 0.130 -> 0.123 ms at M4 1024^2)
-    constexpr bool SREAD = ASYNC;
     CT* stage = reinterpret_cast<CT*>(twPl + 2 * MM + 1);               // [3 XTL] next NL panel
 
     const Geo g = bt.geo[blockIdx.z];
@@ -1536,28 +1535,18 @@ __global__ __launch_bounds__(xs_of<LXT>(), 3) void k_xstep(Batch bt, const cplx_
             asm volatile("" : "+v"(tidv));
             if constexpr (ASYNC) {
                 // this line's panel has landed in the staging area.  A whole
-                // tile's transforms read it there (MM <= 512); otherwise it is
-                // laid out for them first, and the next line's panel starts then
+                // tile's transforms read it there; otherwise it is laid out for
+                // them first, and the next line's panel starts then
                 wait_vmem();
                 __syncthreads();
-                if (!(SREAD && whole)) {
-                    if (whole) {
-                        int t0, xq, pa;
-                        CT* rb;
-                        tile_item(tidv, t0, xq, rb, pa);
-                        static_for<0, LPT>([&](auto qi) {
-                            constexpr int q = decltype(qi)::value;
-                            swz<q * DA>(rb, pa) = stage[tidv + XS * q];
-                        });
-                    } else {
+                if (!whole) {
 #pragma unroll
-                        for (int q = 0; q < LPT; q++) {
-                            const int i = tidv + XS * q;
-                            if (i >= nrows) continue;
-                            const int x = i >> lgNT, t = i & (NT - 1);
-                            const int a = x / 3, b = x - 3 * a;
-                            reg[(t * 3 + b) * MM + (pidx(a) ^ xsw<R>(t, b))] = stage[i];
-                        }
+                    for (int q = 0; q < LPT; q++) {
+                        const int i = tidv + XS * q;
+                        if (i >= nrows) continue;
+                        const int x = i >> lgNT, t = i & (NT - 1);
+                        const int a = x / 3, b = x - 3 * a;
+                        reg[(t * 3 + b) * MM + (pidx(a) ^ xsw<R>(t, b))] = stage[i];
                     }
                     __syncthreads();
                     int ln = li + 1;
@@ -1605,7 +1594,7 @@ __global__ __launch_bounds__(xs_of<LXT>(), 3) void k_xstep(Batch bt, const cplx_
             if (seq_on) {
                 CT v[PL];
                 const int pg = pidx(gl) ^ sxo;
-                if (SREAD && whole) {
+                if (ASYNC && whole) {
                     // element a of sequence (t, b) = (s/3, s%3) is panel row
                     // x = 3a + b, column t of the staged panel
                     const CT* sb = stage + (3 * gl + s % 3) * NTC + s / 3;
@@ -1613,13 +1602,13 @@ __global__ __launch_bounds__(xs_of<LXT>(), 3) void k_xstep(Batch bt, const cplx_
                 } else {
                     static_for<0, PL>([&](auto qi) { v[qi] = swz<decltype(qi)::value * G>(myreg, pg); });
                 }
-                if constexpr (BLK && !SREAD) __syncthreads();
+                if constexpr (BLK && !ASYNC) __syncthreads(); // at MM = 1024 every tile is whole
                 group_fft<CT, LOGMM, -1, true, 7, 1, 0, 0, BLK>(v, myreg, gl, twMl, sxo);
                 if constexpr (BLK) __syncthreads();
                 static_for<0, PL>([&](auto qi) { swz<decltype(qi)::value * G>(myreg, pg) = v[qi]; });
             }
             __syncthreads();
-            if constexpr (SREAD) {
+            if constexpr (ASYNC) {
                 if (whole) { // the staged panel has been read: start the next line's
                     int ln = li + 1;
                     while (ln < NLI && !line_on(ln)) ln++;

@@ -195,7 +195,7 @@ struct SizeClass {
     double2 *twMMd = nullptr, *twNNd = nullptr, *twPd = nullptr, *twQd = nullptr;
     float2 *twMMf = nullptr, *twNNf = nullptr, *twQf = nullptr;
     int nst = 1;
-    bool u_valid = false; // U holds the x-inverse of the current c (with the laminar profile)
+    bool u_valid = false; // U holds the x-inverse of the current c (advective form: with the laminar profile)
     Plan base;            // the rule-based plan; plan = base with the chosen alternatives
     int choice = 0;       // autotuner choice bits (see g_tune_cache)
 
@@ -258,8 +258,12 @@ struct SizeClass {
     // = 256 FP64 146 and 97 us, 1024 x 128 modes mixed 84 and 38 us; M6 2048^2
     // FP64 5140 and 3140 us), its z kernel with two buffers for rows too long for
     // the one-batch kernel (NN = 512: FP64 151 and 141 us with one and two, FP32 74
-    // and 71) and for many rows of 256 points (MM = 256, 1024, one batch and two
-    // buffers: FP64 M4 44 and 52, 161 and 148; FP32 M6 41 and 43, 157 and 117).
+    // and 71) and for x-rows of 256 points where a model has 1536 or more (MM = 256,
+    // 1024, one batch and two buffers: FP64 M4 44 and 52, 161 and 148; FP32 M6 41 and
+    // 43, 157 and 117).  The line is drawn at the size, not at the rows of a launch,
+    // though many members of MM = NN = 256 would gain from two buffers too: the two
+    // kernels differ in rounding, and a member of an ensemble steps to the same bits
+    // as the model alone.
     int rule() const
     {
         if (!base.zc) return 0;

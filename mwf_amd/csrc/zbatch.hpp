@@ -7,7 +7,7 @@
 // block of K0 NN threads (at most 1024) takes one x-row and does each stage of
 // the pass once: fold of all base lines, their inverse transforms, one point
 // per thread for the products, the forward transforms of all rows, and one
-// (k, n) per thread for the lines, with five block barriers in all.
+// (k, n) per thread for the lines, with six block barriers in all.
 //
 // Sequences: inverse (pair p of base lines, phase b) at 3 p + b.  Forward: k = 0
 // (uw, ww - uu) at b; k >= 1 from 3 + 8 (k-1): (uv, uw) at b, (vv - uu, vv - ww) at 3
