@@ -1132,21 +1132,22 @@ __device__ __forceinline__ void s2m_finish(int k, int mi, int n, double2 u, doub
 // Flux form: the share of line type li (fluxline.hpp; not yet scaled, dev_scale)
 // in psi_k and phi_k of the nonlinear term at one (m, n), from the line's forward
 // x transform X.  At (0,0), where every weight vanishes, the mean-mode rows of
-// var_spec2mpt apply instead: psi = -N_u = -ak uv, phi = -N_w = -ak vw = i B.
-__device__ __forceinline__ void dev_term(int li, bool mean, double2 X, double am1, double an1, double ak1, double2& psi,
-                                         double2& phi)
+// var_spec2mpt apply instead: psi = -N_u = -ak uv, phi = -N_w = -ak vw = i B /
+// ak.  rak = 1/ak1, for k = 0 -1.
+__device__ __forceinline__ void dev_term(int li, bool mean, double2 X, double am1, double an1, double ak1, double rak,
+                                         double2& psi, double2& phi)
 {
 #pragma clang fp contract(off)
     if (li == DEV_UV) X = double2{-X.y, X.x}; // i uv
     double cp, cq;
-    dev_weights(li, am1, an1, ak1, cp, cq);
+    dev_weights(li, am1, an1, ak1, rak, cp, cq);
     psi.x = __builtin_fma(cp, X.x, psi.x);
     psi.y = __builtin_fma(cp, X.y, psi.y);
     phi.x = __builtin_fma(cq, X.x, phi.x);
     phi.y = __builtin_fma(cq, X.y, phi.y);
     if (mean) {
         if (li == DEV_UV) psi = double2{-(ak1 * X.y), ak1 * X.x}; // -ak uv, X = i uv
-        if (li == DEV_F) phi = double2{-X.y, X.x};
+        if (li == DEV_F) phi = double2{-(X.y * rak), X.x * rak};
     }
 }
 
@@ -1264,7 +1265,7 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
     const int k = blockIdx.y;
     const int tid = threadIdx.x;
     const int nitems = NT * MM;
-    const double ak1 = ak1_of(k, g.beta);
+    const double ak1 = ak1_of(k, g.beta), rak = k == 0 ? -1.0 : 1.0 / ak1;
 
     // flux form: psi[] and phi[] sum the lines' shares; otherwise psi[] holds
     // u_k until w_k arrives, phi[] holds v_k (am2+an2) until then
@@ -1317,7 +1318,7 @@ __global__ __launch_bounds__(XT) void k_xfwd(Batch bt, const cplx_t<R>* __restri
                 zwave(g, n, an1, an2);
                 const double2 X = X0;
                 if constexpr (FLUX) {
-                    dev_term(li, mi == 0 && n == 0, X, am1, an1, ak1, psi[q][h], phi[q][h]);
+                    dev_term(li, mi == 0 && n == 0, X, am1, an1, ak1, rak, psi[q][h], phi[q][h]);
                     continue;
                 }
                 // var_spec2mpt (program/variables.f90:440-480)
@@ -1501,7 +1502,7 @@ __global__ __launch_bounds__(xs_of<LXT>(), 3) void k_xstep(Batch bt, const cplx_
         rb = reg + (t0 * 3 + b0) * MM;
         pa = pidx(a0) ^ xsw<R>(t0, b0);
     };
-    const double ak1 = ak1_of(k, g.beta);
+    const double ak1 = ak1_of(k, g.beta), rak = k == 0 ? -1.0 : 1.0 / ak1;
     const double ak2 = ak2_of(k, g.beta);
 
     // flux form: psi[] and phi[] sum the lines' shares; otherwise psi[] holds
@@ -1634,7 +1635,7 @@ __global__ __launch_bounds__(xs_of<LXT>(), 3) void k_xstep(Batch bt, const cplx_
                     xwave(g, mi, am1, am2);
                     zwave(g, n, an1, an2);
                     if constexpr (FLUX) {
-                        dev_term(li, mi == 0 && n == 0, X, am1, an1, ak1, psi[q][h], phi[q][h]);
+                        dev_term(li, mi == 0 && n == 0, X, am1, an1, ak1, rak, psi[q][h], phi[q][h]);
                         continue;
                     }
                     if (li == 0) {

@@ -46,7 +46,7 @@ __global__ __launch_bounds__(xa_threads<LOGXA>()) void k_xall(Batch bt, const cp
     const int n0 = xcd_tile(blockIdx.x, gridDim.x) << LOGNT;
     const int k = blockIdx.y;
     const int tid = threadIdx.x;
-    const double ak1 = ak1_of(k, g.beta);
+    const double ak1 = ak1_of(k, g.beta), rak = k == 0 ? -1.0 : 1.0 / ak1;
     const double ak2 = ak2_of(k, g.beta);
     const int nlin = k == 0 ? 2 : 4; // NL lines
 
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(xa_threads<LOGXA>()) void k_xall(Batch bt, const cp
                     double am1, am2, an1, an2;
                     xwave(g, mi, am1, am2);
                     zwave(g, n, an1, an2);
-                    dev_term(l, mi == 0 && n == 0, h == 0 ? Xp : Xn, am1, an1, ak1, psi[h], phi[h]);
+                    dev_term(l, mi == 0 && n == 0, h == 0 ? Xp : Xn, am1, an1, ak1, rak, psi[h], phi[h]);
                 }
             }
             const double dt = g.dt;

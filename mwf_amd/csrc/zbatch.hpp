@@ -190,7 +190,7 @@ __global__ __launch_bounds__((zs_threads<K0, LOGNN>())) void k_zs(Batch bt, cons
             CT d;
             pair(buf, uw, d);
             st_piece(nlr + DEV_UW * nls, uw, wide);
-            st_piece(nlr + DEV_F * nls, cscale(d, (R)-gn), wide);
+            st_piece(nlr + DEV_F * nls, cscale(d, (R)gn), wide);
             continue;
         }
         const CT* sk = buf + (3 + 8 * (k - 1)) * LPZ;
@@ -203,9 +203,9 @@ __global__ __launch_bounds__((zs_threads<K0, LOGNN>())) void k_zs(Batch bt, cons
         vw = cadd(vw, cmul(a, w1));
         split(sk + 7 * LPZ, a, c);
         vw = cadd(vw, cmul(a, w2));
-        const DevMul<R> m = dev_mul<R>(gn, ak1_of(k, g.beta));
+        const DevMul<R> m = dev_mul<R>(gn, 1.0 / gn, ak1_of(k, g.beta));
         if (m.far) vvuu = csub(vvuu, vvww); // ww - uu
         st_piece(nlr + DEV_F * nls, CT{m.f * vvww.x - m.h * vw.y, m.f * vvww.y + m.h * vw.x}, wide);
-        st_piece(nlr + DEV_E * nls, CT{vvuu.x + m.e * vw.y, vvuu.y - m.e * vw.x}, wide);
+        st_piece(nlr + DEV_E * nls, CT{m.ak * vvuu.x + m.e * vw.y, m.ak * vvuu.y - m.e * vw.x}, wide);
     }
 }

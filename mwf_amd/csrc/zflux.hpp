@@ -72,7 +72,7 @@ template <int K0_, int PART = 0> struct Dev {
         return 2 + 5 * (q / 2) + (PART == 2 ? (q & 1 ? VVUU : UV) : (q & 1 ? VVWW : VW));
     }
     // uses of row r: line, kind
-    enum { ROW, NEG_G, VW_E, VW_F, WW_E, WW_F }; // row, -g row, and the multiples of DevMul
+    enum { ROW, G_ROW, UU_E, VW_E, VW_F, WW_E, WW_F }; // row, g row, and the multiples of DevMul
     __host__ __device__ static constexpr int nuse(int r) { return type(r) == VW || type(r) == VVWW ? 2 : 1; }
     __host__ __device__ static constexpr int use_line(int r, int u)
     {
@@ -84,7 +84,7 @@ template <int K0_, int PART = 0> struct Dev {
     __host__ __device__ static constexpr int use_kind(int r, int u)
     {
         const int t = type(r);
-        return t == WWUU ? NEG_G : t == VW ? (u == 0 ? VW_E : VW_F) : t == VVWW ? (u == 0 ? WW_E : WW_F) : ROW;
+        return t == WWUU ? G_ROW : t == VVUU ? UU_E : t == VW ? (u == 0 ? VW_E : VW_F) : t == VVWW ? (u == 0 ? WW_E : WW_F) : ROW;
     }
     // forward positions of the first and the last row of line L
     __host__ __device__ static constexpr int first(int L)
@@ -326,7 +326,6 @@ __device__ __forceinline__ void zc_pass(const Geo& g, int xt, const cplx_t<R>* _
 
     // ---- products, forward z transforms (r2c, -1), line assembly ----
     const double gn = g.gamma * r, rgn = 1.0 / gn; // gamma n at the thread's output n = r
-    const double rbeta = 1.0 / g.beta;
     const R lu = (R)g.cth, lw = (R)g.sth; // laminar u_1, w_1
     if constexpr (HT) {
         tf[0] = cconj(twQl[r]);
@@ -350,12 +349,13 @@ __device__ __forceinline__ void zc_pass(const Geo& g, int xt, const cplx_t<R>* _
                     constexpr int L = FX::use_line(row, u), kind = FX::use_kind(row, u);
                     constexpr int k = FX::k(row);
                     CT term = xs;
-                    if constexpr (kind == FX::NEG_G) term = cscale(xs, (R)-gn);
+                    if constexpr (kind == FX::G_ROW) term = cscale(xs, (R)gn);
                     else if constexpr (kind != FX::ROW) {
-                        const DevMul<R> m = dev_mul<R>(gn, rgn, ak1_of(k, g.beta), (k & 1 ? -1.0 : 1.0) / k * rbeta);
+                        const DevMul<R> m = dev_mul<R>(gn, rgn, ak1_of(k, g.beta));
                         if constexpr (kind == FX::VW_E) term = CT{xs.y * m.e, -(xs.x * m.e)};
                         else if constexpr (kind == FX::VW_F) term = CT{-(xs.y * m.h), xs.x * m.h};
-                        else if constexpr (kind == FX::WW_E) term = m.far ? CT{-xs.x, -xs.y} : CT{(R)0, (R)0};
+                        else if constexpr (kind == FX::UU_E) term = cscale(xs, m.ak);
+                        else if constexpr (kind == FX::WW_E) term = cscale(xs, m.far ? -m.ak : (R)0);
                         else term = cscale(xs, m.f);
                     }
                     if constexpr (FX::first(L) == q) acc[L] = term;

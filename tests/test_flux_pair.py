@@ -23,15 +23,16 @@ def lib(tmp_path_factory):
     src, so = d / "line.cpp", d / "line.so"
     src.write_text("#define __host__\n#define __device__\n"
                    f'#include "{csrc}/fluxline.hpp"\n'
-                   'template <typename M> static void put(M m, double* o) { o[0] = m.e; o[1] = m.f; o[2] = m.h; o[3] = m.far; }\n'
-                   'extern "C" void mul(double g, double ak, int rcp, int single, double* o) {\n'
-                   "  if (single) put(rcp ? dev_mul<float>(g, 1 / g, ak, 1 / ak) : dev_mul<float>(g, ak), o);\n"
-                   "  else put(rcp ? dev_mul<double>(g, 1 / g, ak, 1 / ak) : dev_mul<double>(g, ak), o);\n}\n"
-                   'extern "C" void weights(int li, double a, double g, double ak, double* o) { dev_weights(li, a, g, ak, o[0], o[1]); }\n')
+                   'template <typename M> static void put(M m, double* o) { o[0] = m.ak; o[1] = m.e; o[2] = m.f; o[3] = m.h; o[4] = m.far; }\n'
+                   'extern "C" void mul(double g, double ak, int single, double* o) {\n'
+                   "  if (single) put(dev_mul<float>(g, 1 / g, ak), o);\n"
+                   "  else put(dev_mul<double>(g, 1 / g, ak), o);\n}\n"
+                   'extern "C" void weights(int li, double a, double g, double ak, double* o) {\n'
+                   "  dev_weights(li, a, g, ak, ak == 0 ? -1.0 : 1 / ak, o[0], o[1]);\n}\n")
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-Wno-unknown-pragmas", "-o", str(so), str(src)], check=True)
     L = ctypes.CDLL(str(so))
     dp, cd, ci = ctypes.POINTER(ctypes.c_double), ctypes.c_double, ctypes.c_int
-    L.mul.argtypes, L.weights.argtypes = [cd, cd, ci, ci, dp], [ci, cd, cd, cd, dp]
+    L.mul.argtypes, L.weights.argtypes = [cd, cd, ci, dp], [ci, cd, cd, cd, dp]
     return L
 
 
@@ -51,8 +52,7 @@ def _psi_phi(lib, lines, a, g, ak):
     return psi, phi
 
 
-@pytest.mark.parametrize("rcp", [0, 1])
-def test_single_precision_lines_keep_the_precision_of_the_terms(lib, rcp):
+def test_single_precision_lines_keep_the_precision_of_the_terms(lib):
     """Rows of unit size.  Each line is a sum of up to three shares (row times
     multiplier), a share with at most three roundings and a sum with two: 5 u of the
     sum of its shares.  By |g| <= |ak| or |g| > |ak| the weighted shares are at most
@@ -66,12 +66,12 @@ def test_single_precision_lines_keep_the_precision_of_the_terms(lib, rcp):
         if rng.random() < 0.1:
             g = ak * rng.choice([-1, 1]) * (1 + rng.choice([0.0, 1e-9, -1e-9]))
         uv, uw, vvuu, vw, vvww = (rng.uniform(-1, 1, 5) + 1j * rng.uniform(-1, 1, 5)).astype(np.complex64)
-        e, f, h, far = _call(lib.mul, 4, g, ak, rcp, 1)
+        akr, e, f, h, far = _call(lib.mul, 5, g, ak, 1)
         assert bool(far) == (abs(g) > abs(ak))
-        e, f, h = (np.float32(x) for x in (e, f, h))
-        assert np.isfinite([e, f, h]).all()
+        akr, e, f, h = (np.float32(x) for x in (akr, e, f, h))
+        assert np.isfinite([akr, e, f, h]).all()
         x = vvuu - vvww if far else vvuu
-        lines = {UW: uw, UV: uv, E: np.complex64(complex(np.float32(x.real + e * vw.imag), np.float32(x.imag - e * vw.real))),
+        lines = {UW: uw, UV: uv, E: np.complex64(complex(np.float32(akr * x.real + e * vw.imag), np.float32(akr * x.imag - e * vw.real))),
                  F: np.complex64(complex(np.float32(f * vvww.real - h * vw.imag), np.float32(f * vvww.imag + h * vw.real)))}
         psi, phi = _psi_phi(lib, lines, a, g, ak)
         uv, uw, vvuu, vw, vvww = (complex(x) for x in (uv, uw, vvuu, vw, vvww))
@@ -111,18 +111,18 @@ def test_lines_and_weights_give_the_nonlinear_term(lib, k0, mm, nn, theta, alpha
             uv, uw, vvuu, vw, vvww = np.moveaxis(_from_xz(o, np.stack(rows, axis=2)), 2, 0)
         for n in range(o.nn):
             g = float(kz[n, 0, 0])
-            e, f, h, far = _call(lib.mul, 4, g, ak if k else 1.0, 0, 0)
+            _, e, f, h, far = _call(lib.mul, 5, g, ak if k else 1.0, 0)
             for mi in range(o.M):
                 a, at = float(kx[0, mi, 0]), (n, mi)
                 if k == 0:
                     w = [_call(lib.weights, 2, li, a, g, 0.0)[0] for li in (UW, F)]
-                    got[n, mi, 0] = w[0] * uw[at] + w[1] * (-g * wwuu[at])
+                    got[n, mi, 0] = w[0] * uw[at] + w[1] * (g * wwuu[at])
                     continue
-                lines = {UW: uw[at], UV: uv[at], E: vvuu[at] - 1j * e * vw[at] - (vvww[at] if far else 0),
+                lines = {UW: uw[at], UV: uv[at], E: ak * (vvuu[at] - (vvww[at] if far else 0)) - 1j * e * vw[at],
                          F: f * vvww[at] + 1j * h * vw[at]}
                 psi, phi = _psi_phi(lib, lines, a, g, ak)
                 if n == 0 and mi == 0:
-                    psi, phi = -ak * uv[at], 1j * lines[F]
+                    psi, phi = -ak * uv[at], 1j * lines[F] / ak
                 got[n, mi, k], got[n, mi, k0 - 1 + k] = psi, phi
     got[0, 0, 0] = 0
     scale = max(np.abs(want[0]).max(), np.abs(want[1]).max())
