@@ -13,13 +13,13 @@
 //
 // A line is rounded to the precision of the transforms before its weight is
 // applied, so no weighted part of a line may be large and cancel.  Of A, B the
-// parts a (g^2 / ak) vw cancel in psi, of C, D the parts a^2 (ak^2 / g) vw and ak^2 g
-// vw in phi: harmless where |g| <= |ak| and where |g| > |ak| respectively, g / ak and
-// more times the result's own rounding elsewhere.  So the pair is chosen per n: C, D
+// parts a (g^2 / ak) vw cancel in psi, of C, D the parts a^2 (ak^2 / g) vw in phi:
+// harmless where |g| <= |ak| and where |g| > |ak| respectively, g / ak and ak / g times
+// the result's own rounding elsewhere.  So the pair is chosen per n: C, D
 // where |g| > |ak| (far), else A, B.  The first line has the same weights in both.
 // With A and B throughout, the nonlinear term of a full spectrum with alpha
 // MM = gamma NN = 4096 was off by 9.3e-6 in FP32 and 2.1e-14 in FP64 (MM = NN = 32),
-// with the rule by 1.9e-7 and 4.9e-16, and at every box it is closer in FP32 than the
+// with the rule by 1.9e-7 and 4.9e-16, and at every box tried it is closer in FP32 than the
 // form with a line per velocity component (alpha MM = gamma NN = 512, evaluated on
 // the CPU: 1.6e-7 and 2.4e-7; 8: 1.7e-7 and 3.3e-7).  It costs the z kernels up to
 // 1.5 % (FP64 M6 NN = 512, 211 -> 214 us).

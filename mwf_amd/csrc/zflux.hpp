@@ -63,11 +63,22 @@ template <int K0_, int PART = 0> struct Dev {
     enum { UV, UW, VVUU, VW, VVWW, WWUU };
     __host__ __device__ static constexpr int k(int r) { return r < 2 ? 0 : 1 + (r - 2) / 5; }
     __host__ __device__ static constexpr int type(int r) { return r < 2 ? (r == 0 ? UW : WWUU) : (r - 2) % 5; }
-    // row at forward position q (two per complex sequence), -1 = padding
+    // row at forward position q (two per complex sequence), -1 = padding.  Rounded
+    // twiddles leak a few 1e-8 of one row of a sequence into the other in FP32, alike in
+    // every step.  At small a and g, psi weights uv and vw by ak, uw and uu by a and g only,
+    // and the laminar profile makes uw and uu the larger rows: so uv and vw share a
+    // sequence, and vw does not share uu's.  (State after 50 steps against FP64, with uv, uw /
+    // vv - uu, vw / ... and now: M6 MM = 64, NN = 1024 6.4e-8 and 5.7e-8, NN = 512 5.1e-8 and
+    // 4.7e-8, M6 2048^2 7.7e-8 and 6.9e-8; the advective form 6.0e-8, 6.3e-8 for the first
+    // two.)  The three lines' worth of vw, vv - ww and vv - uu follow one another, so that
+    // few accumulators are live.
     __host__ __device__ static constexpr int order(int q)
     {
         if (q >= NR) return -1;
-        if (PART == 0) return q;
+        if (PART == 0) {
+            constexpr int odd[] = {UV, VW, VVWW, VVUU, UW}, even[] = {UW, UV, VW, VVWW, VVUU};
+            return q < 2 ? q : 2 + 5 * ((q - 2) / 5) + (((q - 2) / 5) % 2 ? even : odd)[(q - 2) % 5];
+        }
         if (PART == 1) return q < 2 ? q : 2 + 5 * (q - 2) + UW;
         return 2 + 5 * (q / 2) + (PART == 2 ? (q & 1 ? VVUU : UV) : (q & 1 ? VVWW : VW));
     }
