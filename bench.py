@@ -312,6 +312,8 @@ PROFILE_CASES = {
     "m4_1024": (WORKLOAD, IC),
     "m6_2048": (dict(k0=6, mm=1024, nn=1024, lx=256 * np.pi, lz=256 * np.pi, re=250.0, dt=0.01),
                 dict(seed=3, scl=0.3, k0=8.0)),
+    "m6_256": (dict(k0=6, mm=128, nn=128, lx=32 * np.pi, lz=32 * np.pi, re=200.0, dt=0.02), dict(seed=1, scl=0.3, k0=8.0)),
+    "m4_1024x128": (dict(k0=4, mm=512, nn=64, lx=128 * np.pi, lz=16 * np.pi, re=200.0, dt=0.02), dict(seed=1, scl=0.3, k0=8.0)),
 }
 
 

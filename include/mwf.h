@@ -159,7 +159,8 @@ int mwf_blend(mwf_handle *a, mwf_handle *b, double d, mwf_handle *dst);
 
 /* Autotuning, in place of tra_precompute's FFTW_PATIENT planning
  * (program/transform.fftw5.f90:33-59).  Process-wide mode for handles and
- * ensembles created afterwards: 0 (default) = rule-based plans; 1 = the first
+ * ensembles created afterwards: 0 (default) = rule-based plans (the flux form,
+ * bit 3 below, by the size alone); 1 = the first
  * handle or ensemble class of each (precision, k0, mm, nn) times its
  * candidate kernel plans at creation (a few steps each, on its zero state)
  * and keeps the fastest, and later ones of that size reuse the choice, so
@@ -172,7 +173,10 @@ int mwf_autotune(int32_t mode);
  * thread (768-thread blocks) instead of three (512), bit 3 = the flux
  * (conservative) form of vel_nonlinear's products: the same projected
  * (u.grad)u, with d/dx, d/dz taken in spectral space and d/dy moved onto the
- * wall-normal bases, equal to the advective form up to rounding; bit 4 (with
+ * wall-normal bases, equal to the advective form up to rounding (which the
+ * flux form amplifies at wavenumbers far above those the field fills: where
+ * alpha mm or gamma nn is far above 10, mode 2, the advective form, gives the
+ * term itself more precisely); bit 4 (with
  * bit 3) = its z kernel with two LDS buffers, a barrier per batch fewer;
  * bit 5 (advective form, NN = 1024; implies bit 1 in the mixed form) = the
  * phase-sequential z kernel with the three fold phases of an x-row in three
