@@ -194,7 +194,7 @@ struct HostStage {
         nslot = most > CHUNK ? NSLOT : 1;
         chunk = std::min(CHUNK, (most + 4095) / 4096 * 4096);
         pool = CopyPool::get();
-        hipError_t e = hipHostMalloc((void**)&buf, chunk * nslot, hipHostMallocDefault);
+        hipError_t e = hipHostMalloc((void**)&buf, chunk * nslot, hipHostMallocCoherent); // kernels access it too (DIRECT)
         for (int i = 0; i < nslot && e == hipSuccess; i++) e = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming);
         return e;
     }
