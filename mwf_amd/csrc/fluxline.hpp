@@ -22,7 +22,9 @@
 // with the rule by 1.9e-7 and 4.9e-16, and at every box tried it is closer in FP32 than the
 // form with a line per velocity component (alpha MM = gamma NN = 512, evaluated on
 // the CPU: 1.6e-7 and 2.4e-7; 8: 1.7e-7 and 3.3e-7).  It costs the z kernels up to
-// 1.5 % (FP64 M6 NN = 512, 211 -> 214 us).
+// 1.5 % (FP64 M6 NN = 512, 211 -> 214 us), a step at most 1 % but for short launches of
+// FP64 rows of 512 (M4 MM = 128, 87.6 -> 90.6 us), and the one-buffer FP64 form, which no
+// rule picks, the registers it has not got (M4 MM = NN = 512, k_zc 152 -> 191 us).
 // For k = 0: uw and B = g (ww - uu), psi = (a^2 - g^2) uw + a B.
 #pragma once
 

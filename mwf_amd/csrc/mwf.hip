@@ -257,8 +257,8 @@ struct SizeClass {
     // The rule-based choice: the flux form (M4 steps, advective and flux: MM = NN
     // = 256 FP64 146 and 97 us, 1024 x 128 modes mixed 84 and 38 us; M6 2048^2
     // FP64 5140 and 3140 us), its z kernel with two buffers for rows too long for
-    // the one-batch kernel (NN = 512: FP64 151 and 141 us with one and two, FP32 74
-    // and 71) and for x-rows of 256 points where a model has 1536 or more (MM = 256,
+    // the one-batch kernel (NN = 512: FP64 191 and 134 us with one and two, FP32 75
+    // and 69) and for x-rows of 256 points where a model has 1536 or more (MM = 256,
     // 1024, one batch and two buffers: FP64 M4 44 and 52, 161 and 148; FP32 M6 41 and
     // 43, 157 and 117).  The line is drawn at the size, not at the rows of a launch,
     // though many members of MM = NN = 256 would gain from two buffers too: the two

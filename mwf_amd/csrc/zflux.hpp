@@ -36,8 +36,8 @@
 
 // Rows and lines of the z pass.  Row r (value: FluxRows in flux_gen.hpp): 0, 1
 // are uw_0, ww_0 - uu_0; 2 + 5 (k-1) + t, t = 0..4, are uv, uw, vv - uu, vw, vv -
-// ww of k >= 1, transformed two per complex sequence in this order.  Lines of
-// k start at dev_line(k).
+// ww of k >= 1, transformed two per complex sequence in the order of order().
+// Lines of k start at dev_line(k).
 //
 // U holds the perturbation; the laminar profile enters where the rows are
 // formed, without its own products, whose constants only the unused (0,0) modes

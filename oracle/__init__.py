@@ -1,6 +1,6 @@
 """CPU restatement of the reference per-step path -- the oracle.
 
-TEST INFRASTRUCTURE ONLY.  This package is the checker for the HIP library in
+TEST INFRASTRUCTURE ONLY.  This package is the oracle of the HIP library in
 ``mwf_amd``: only ``tests/``, ``__graft_entry__.smoke()`` and the
 ``cpu_baseline`` leg of ``bench.py`` may import it.  The product never does.
 

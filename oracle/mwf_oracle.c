@@ -1,7 +1,7 @@
 /*
  * mwf_oracle.c -- CPU restatement of the Model Waleffe Flow per-step path.
  *
- * TEST INFRASTRUCTURE ONLY: the checker for the HIP library (see the header).
+ * TEST INFRASTRUCTURE ONLY: the oracle of the HIP library (see the header).
  *
  * Each routine below restates one reference routine, cited as file:line
  * relative to the reference root, in the same loop order and with the same

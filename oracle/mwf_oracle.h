@@ -1,7 +1,7 @@
 /*
  * mwf_oracle.h -- CPU restatement of the Model Waleffe Flow per-step path.
  *
- * TEST INFRASTRUCTURE ONLY.  This is the checker for the HIP library in
+ * TEST INFRASTRUCTURE ONLY.  This is the oracle of the HIP library in
  * mwf_amd/.  Only tests/, __graft_entry__.smoke() and the cpu_baseline leg of
  * bench.py load it, and only to check or to time the CPU path; the product
  * library never links or calls it.
